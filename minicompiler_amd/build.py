@@ -67,7 +67,8 @@ EMBEDDED = {"kGemmF32MfmaSource": CSRC / "hip" / "gemm_f32_mfma.h",
             "kGemmF32RingSource": CSRC / "hip" / "gemm_f32_ring.h",
             "kGemmF32NarrowSource": CSRC / "hip" / "gemm_f32_narrow.h",
             "kGemmSplitArrivalSource": CSRC / "hip" / "gemm_split_arrival.h",
-            "kGemm16FastSource": CSRC / "hip" / "gemm_mfma16_fast.h"}
+            "kGemm16FastSource": CSRC / "hip" / "gemm_mfma16_fast.h",
+            "kGemm16FragSource": CSRC / "hip" / "gemm_mfma16_frag.h"}
 
 
 def _embed() -> Path:

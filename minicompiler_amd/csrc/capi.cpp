@@ -773,6 +773,10 @@ MC_API int mc_generate_gemm_epilogue_kernel(const char* program, int acc_input, 
         {"narrow64", hip::GemmBody::F32Narrow64, &hip::kGemmF32NarrowSource},
         {"bf16", hip::GemmBody::Bf16Fast, &hip::kGemm16FastSource},
         {"f16", hip::GemmBody::F16Fast, &hip::kGemm16FastSource},
+        {"bf16_packed", hip::GemmBody::Bf16Packed, &hip::kGemm16FastSource},
+        {"f16_packed", hip::GemmBody::F16Packed, &hip::kGemm16FastSource},
+        {"bf16_frag", hip::GemmBody::Bf16Frag, &hip::kGemm16FastSource},
+        {"f16_frag", hip::GemmBody::F16Frag, &hip::kGemm16FastSource},
     };
     const BodyName* chosen = nullptr;
     const std::string want = body && *body ? body : "two_stage";

@@ -18,6 +18,7 @@
 
 #include "codegen.hpp"
 
+#include "matmul.h"
 #include "rtc_sources.hpp"
 
 #include <algorithm>
@@ -287,7 +288,7 @@ GemmEpilogueKernel generate_gemm_epilogue_kernel(const FusedProgram& program, st
                                                  GemmBody body, const GemmDims& fixed) {
     const std::size_t num_inputs = input_shapes.size();
     std::ostringstream os;
-    os << "// minicompiler-hip " << (is_f32_body(body) ? "FP32" : body == GemmBody::Bf16Fast ? "bf16" : "fp16")
+    os << "// minicompiler-hip " << (is_f32_body(body) ? "FP32" : is_bf16_body(body) ? "bf16" : "fp16")
        << " GEMM with a fused epilogue: " << program.num_ops() << " op(s) on the result, out f32"
        << to_string(out_shape) << ".\n";
     // The ring and narrow bodies add split-K partials in the launch through
@@ -295,6 +296,7 @@ GemmEpilogueKernel generate_gemm_epilogue_kernel(const FusedProgram& program, st
     const bool folds = is_f32_body(body) && body != GemmBody::F32Mfma;
     if (folds) os << kGemmSplitArrivalSource << "\n";
     os << gemm_body_source << "\n";
+    if (is_frag_body(body)) os << kGemm16FragSource << "\n";
     os << program_function(program, num_inputs);
     // Index helpers of General inputs, in terms of the flat output index i.
     for (std::size_t k = 0; k < num_inputs; ++k) {
@@ -334,12 +336,23 @@ GemmEpilogueKernel generate_gemm_epilogue_kernel(const FusedProgram& program, st
                                        : std::string("k_split, depth");
     const char* unused = constant ? "\t(void)m;\n\t(void)n;\n\t(void)k;\n" : "";
     if (!is_f32_body(body)) {
-        // `a` is packed A (the graph rounds and packs it, mc_convert_pack_a_f32).
-        os << "extern \"C\" __global__ void __launch_bounds__(512, 1)\n" << kGemmEpilogueKernelName
+        // `a` is packed A (the graph rounds and packs it), and `b` packed B for the packed and frag bodies.
+        const char* type = is_bf16_body(body) ? "true" : "false";
+        std::string call, bounds = "512, 1";
+        if (is_frag_body(body)) {
+            bounds = std::to_string(mchip_frag_threads(fixed.frag));
+            call = std::string("mc_gemm16_frag<") + type + ", McFragCfg<" +
+                   std::to_string(mchip_frag_rows(fixed.frag) / 16) + ", " +
+                   std::to_string(mchip_frag_cols(fixed.frag) / 16) + ">>";
+        } else if (body == GemmBody::Bf16Packed || body == GemmBody::F16Packed) {
+            call = std::string("mc_gemm16_packed<") + type + ">";
+        } else {
+            call = std::string("mc_gemm16_fast<") + type + ", true>";
+        }
+        os << "extern \"C\" __global__ void __launch_bounds__(" << bounds << ")\n" << kGemmEpilogueKernelName
            << "(const unsigned short* __restrict__ a, const unsigned short* __restrict__ b, float* __restrict__ c, "
               "int m, int n, int k, McEpilogue epi)\n{\n"
-           << unused << "\tmc_gemm16_fast<" << (body == GemmBody::Bf16Fast ? "true" : "false")
-           << ", true>(a, b, c, " << mnk << ", epi);\n}\n";
+           << unused << "\t" << call << "(a, b, c, " << mnk << ", epi);\n}\n";
         return {os.str()};
     }
     const char* bounds = body == GemmBody::F32RingBig || body == GemmBody::F32RingThin ? "256, 1"

@@ -91,7 +91,16 @@ enum class GemmBody {
     F32Narrow64,  // likewise, 64x64 tiles
     Bf16Fast,     // bf16 operands in HBM, 256x256 tiles, 512 lanes, one block per tile
     F16Fast,      // fp16 operands, likewise
+    Bf16Packed,   // bf16, the same tiles, both operands packed
+    F16Packed,    // fp16, likewise
+    Bf16Frag,     // bf16, both operands packed, 16x16 to 64x64 tiles (gemm_mfma16_frag.h)
+    F16Frag,      // fp16, likewise
 };
+
+inline bool is_frag_body(GemmBody body) { return body == GemmBody::Bf16Frag || body == GemmBody::F16Frag; }
+inline bool is_bf16_body(GemmBody body) {
+    return body == GemmBody::Bf16Fast || body == GemmBody::Bf16Packed || body == GemmBody::Bf16Frag;
+}
 
 inline bool is_narrow_body(GemmBody body) {
     return body == GemmBody::F32Narrow16 || body == GemmBody::F32Narrow32 || body == GemmBody::F32Narrow16x64 ||
@@ -131,7 +140,8 @@ inline const char* narrow_config(GemmBody body) {
 // body and `counters` not null (one zeroed unsigned per tile), the GEMM
 // launch adds the partials itself and the sum kernel is not launched; the
 // two-stage body ignores counters. 16-bit bodies (one block of 512 lanes per
-// 256x256 tile): (a, b, c, m, n, k, epi). epi holds one float pointer per program
+// 256x256 tile, or the grid and block of mchip_frag_grid / _threads):
+// (a, b, c, m, n, k, epi), k the padded K where both operands are packed. epi holds one float pointer per program
 // input (that of `acc_input` unused). `vectorized_operands` (FP32): A and B
 // rows allow 16-byte loads (k and n multiples of 4, 16-byte aligned).
 // The product's dimensions, when the kernel serves one shape only: the
@@ -140,6 +150,7 @@ inline const char* narrow_config(GemmBody body) {
 // element) and ignores its m, n, k, k_split and depth arguments.
 struct GemmDims {
     int m = 0, n = 0, k = 0, k_split = 0, depth = 1;
+    int frag = 0;  // Bf16Frag, F16Frag: the tile shape (MCHIP_FRAG_*)
 };
 
 GemmEpilogueKernel generate_gemm_epilogue_kernel(const FusedProgram& program, std::size_t acc_input,

@@ -6,6 +6,7 @@
 #pragma once
 
 typedef float mc_f32x4_t __attribute__((ext_vector_type(4)));
+typedef float mc_f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));  // at any float address
 typedef unsigned short mc_u16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 mc_bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 mc_f16x8_t __attribute__((ext_vector_type(8)));
@@ -89,8 +90,19 @@ typedef short s16x4 __attribute__((ext_vector_type(4)));
 // Element (row, kk) of an M x K matrix sits at index
 //   (row / 256) 256 K + (kk / 32) 8192 + (row % 256 / 16) 512 + (kk % 32 / 8) 128 + (row % 16) 8 + kk % 8.
 // On an MI355X the 8192^3 bf16 product took 787-795 us so against 840-845 us
-// with row-major A (timing copies, one process); the same layout for B
-// gained nothing (B's fetch already reads 512 bytes per k row).
+// with row-major A (timing copies, one process).
+//
+// Packed B (the kPackedB form, which the compiled graphs run): the same layout
+// of B's transpose, 256-column panels of 16 KiB K-step blocks, element (kk, col) at
+//   (col / 256) 256 K + (kk / 32) 8192 + (col % 256 / 16) 512 + (kk % 32 / 8) 128 + (col % 16) 8 + kk % 8.
+// A stage's B region then holds fragments as its A region does: one linear
+// ds_read_b128 per fragment instead of two transposed reads. It is also what
+// makes the kernel's speed independent of the compiler that builds it: hipRTC
+// of ROCm 7.0 (the one a process uses once PyTorch has loaded its own) waits
+// for every load in flight before a transposed read, which serialises the ring.
+// K is padded with zeros to a multiple of 64 in both operands, so any K, N and
+// M run; rows past M and columns past N may hold anything (they only reach C
+// elements that are not stored).
 
 __device__ __forceinline__ int mc_min16(int a, int b) { return a < b ? a : b; }
 #define MC_LDS __attribute__((address_space(3)))
@@ -129,7 +141,7 @@ struct FastLane {
     int a_src[FastShape<kRows>::kFetchA];  // byte offset of the A chunk this lane fetches per instruction (k 0)
     int a_step;                            // bytes between consecutive K steps of A (64 row-major, 16 KiB packed)
     int b_src[2];                          // byte offset of the B chunk (k row 0)
-    int b_step;                            // bytes between consecutive K steps of B
+    int b_step;                            // bytes between consecutive K steps of B (16 KiB packed)
     int a_off[FastShape<kRows>::kRowFrags];  // LDS byte offsets of the A fragments
     int b_off[2][kFColFrags];                // LDS byte offsets of the two transposed B reads
     int wave;
@@ -172,8 +184,9 @@ __device__ __forceinline__ mc_u16x8_t fast_read_a(const MC_LDS unsigned char* rd
     return *reinterpret_cast<const MC_LDS mc_u16x8_t*>(rd + L.a_off[f]);
 }
 
-template <int kRows>
+template <int kRows, bool kPackedB>
 __device__ __forceinline__ mc_u16x8_t fast_read_b(const MC_LDS unsigned char* rd, const FastLane<kRows>& L, int f) {
+    if constexpr (kPackedB) return *reinterpret_cast<const MC_LDS mc_u16x8_t*>(rd + L.b_off[0][f]);
     MC_LDS unsigned char* p = const_cast<MC_LDS unsigned char*>(rd);
     const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<MC_LDS s16x4*>(p + L.b_off[0][f]));
     const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<MC_LDS s16x4*>(p + L.b_off[1][f]));
@@ -185,7 +198,7 @@ __device__ __forceinline__ mc_u16x8_t fast_read_b(const MC_LDS unsigned char* rd
 // middle of the compute phase. `rd` and `wr` are distinct stages;
 // declaring them __restrict__ gives the LDS reads alias scopes that keep the
 // compiler from making them wait for the fetch.
-template <int kRows>
+template <int kRows, bool kPackedB>
 __device__ __forceinline__ void fast_memory_phase(const MC_LDS unsigned char* __restrict__ rd,
                                                   MC_LDS unsigned char* __restrict__ wr, const FastLane<kRows>& L,
                                                   int fetch_k, mc_u16x8_t (&av)[FastShape<kRows>::kRowFrags],
@@ -194,7 +207,7 @@ __device__ __forceinline__ void fast_memory_phase(const MC_LDS unsigned char* __
 #pragma unroll
     for (int f = 0; f < FastShape<kRows>::kRowFrags; ++f) av[f] = fast_read_a<kRows>(rd, L, f);
 #pragma unroll
-    for (int f = 0; f < kFColFrags; ++f) bv[f] = fast_read_b<kRows>(rd, L, f);
+    for (int f = 0; f < kFColFrags; ++f) bv[f] = fast_read_b<kRows, kPackedB>(rd, L, f);
 }
 
 // A workgroup barrier without a memory fence; the compiler may not move
@@ -223,7 +236,9 @@ __device__ __forceinline__ float mc_row_ror8(float x) {
 // a select), after which one register holds rows 0-7 and the other rows
 // 8-15 of the pair, lane l at row 8 h + l % 8 and 16-byte chunk
 // l / 16 + 4 ((l / 8) % 2). Each store instruction then writes 8 whole lines.
-// kCheck: some rows or columns may be past the matrix edge.
+// kCheck: some rows or columns may be past the matrix edge; a chunk of four
+// columns may straddle it (N not a multiple of 4: the 16-byte stores then go
+// to 4-byte aligned addresses).
 // Non-temporal: every CU stores its tile at the same moment, with its matrix
 // units idle until the next tile starts. On one MI355X in one process, at
 // 8192^3 with A packed: 782 us with half-line stores, 766 us with whole
@@ -256,15 +271,23 @@ __device__ __forceinline__ void fast_store(const mc_f32x4_t (&acc)[kRowFrags][kF
                 const unsigned at = static_cast<unsigned>(static_cast<long long>(r) * n + cc);
                 mc_f32x4_t v = t[h];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = epilogue(v[e], at + e);
-                __builtin_nontemporal_store(v, reinterpret_cast<mc_f32x4_t*>(c + static_cast<long long>(r) * n + cc));
+                for (int e = 0; e < 4; ++e)
+                    if (!kCheck || cc + e < n) v[e] = epilogue(v[e], at + e);
+                float* dst = c + static_cast<long long>(r) * n + cc;
+                if (!kCheck || cc + 4 <= n) {
+                    __builtin_nontemporal_store(v, reinterpret_cast<mc_f32x4u_t*>(dst));
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 3; ++e)
+                        if (cc + e < n) __builtin_nontemporal_store(v[e], dst + e);
+                }
             }
         }
     }
 }
 
 // One kRows x 256 tile of C at (row0, col0), all of K.
-template <bool kBf16, int kRows, bool kPackedA, typename Epilogue>
+template <bool kBf16, int kRows, bool kPackedA, bool kPackedB, typename Epilogue>
 __device__ __forceinline__ void fast_tile(MC_LDS unsigned char* lds, const unsigned short* __restrict__ a,
                                           const unsigned short* __restrict__ b, float* __restrict__ c, int m, int n,
                                           int k, int row0, int col0, const Epilogue& epilogue) {
@@ -280,7 +303,8 @@ __device__ __forceinline__ void fast_tile(MC_LDS unsigned char* lds, const unsig
                                       : static_cast<long long>(row0) * k;
     L.a_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(a) + a_base, 0, 0x7fffffff, 0x00020000);
     L.a_step = kPackedA ? kFBM * kFBK * 2 : kFBK * 2;
-    L.b_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(b) + col0, 0, 0x7fffffff, 0x00020000);
+    const long long b_base = kPackedB ? static_cast<long long>(col0) * k : static_cast<long long>(col0);
+    L.b_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<unsigned short*>(b) + b_base, 0, 0x7fffffff, 0x00020000);
     // A: wave w fills the 16-row blocks kFetchA w + i, one per instruction;
     // lane -> (row 16 (kFetchA w + i) + l % 16, chunk l / 16). Rows past the
     // edge are clamped, so every offset is at or past the origin.
@@ -297,15 +321,19 @@ __device__ __forceinline__ void fast_tile(MC_LDS unsigned char* lds, const unsig
         }
     }
     // B: wave w fills k rows 4 w .. 4 w + 3, two per instruction; lane ->
-    // (k row 4 w + 2 i + l / 32, physical chunk l % 32).
+    // (k row 4 w + 2 i + l / 32, physical chunk l % 32). Packed B: as packed A.
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-        const int kr = wave * 4 + i * 2 + (lane >> 5);
-        const int lc = (lane & 31) ^ (2 * swz_b(kr));
-        const int gc = mc_min16(col0 + lc * 8, n - 8);
-        L.b_src[i] = 2 * (kr * n + gc - col0);
+        if constexpr (kPackedB) {
+            L.b_src[i] = (wave * 2 + i) * 1024 + lane * 16;
+        } else {
+            const int kr = wave * 4 + i * 2 + (lane >> 5);
+            const int lc = (lane & 31) ^ (2 * swz_b(kr));
+            const int gc = mc_min16(col0 + lc * 8, n - 8);
+            L.b_src[i] = 2 * (kr * n + gc - col0);
+        }
     }
-    L.b_step = 2 * kFBK * n;
+    L.b_step = kPackedB ? kFBN * kFBK * 2 : 2 * kFBK * n;
     // Wave (wm, wn) of the 2x4 grid owns rows kRows / 2 wm .., columns 64 wn ...
     const int wr = (wave >> 2) * (kRows / 2), wc = (wave & 3) * 64;
     const int g = lane >> 4;
@@ -318,6 +346,10 @@ __device__ __forceinline__ void fast_tile(MC_LDS unsigned char* lds, const unsig
     for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int f = 0; f < kFColFrags; ++f) {
+            if constexpr (kPackedB) {
+                L.b_off[h][f] = kFBOffset + (wc + f * 16) * 64 + lane * 16;
+                continue;
+            }
             const int kr = 8 * g + 4 * h + te;
             const int ncol = wc + f * 16 + 4 * tc;
             const int chunk = (ncol >> 3) ^ (2 * swz_b(kr));
@@ -353,7 +385,7 @@ __device__ __forceinline__ void fast_tile(MC_LDS unsigned char* lds, const unsig
     const int last = (steps - 1) * kFBK;
     for (int t = 0; t < steps; ++t) {
         const int fetch_k = mc_min16((t + 3) * kFBK, last);
-        fast_memory_phase<kRows>(stage(t), stage(t + 3), L, fetch_k, av, bv);
+        fast_memory_phase<kRows, kPackedB>(stage(t), stage(t + 3), L, fetch_k, av, bv);
         __builtin_amdgcn_s_waitcnt(0x0070 | (2 * Sh::kFetch - 2));  // vmcnt(2 kFetch - 2), lgkmcnt(0)
         step_barrier();
 #pragma unroll
@@ -387,9 +419,9 @@ __device__ __forceinline__ void fast_tile(MC_LDS unsigned char* lds, const unsig
 // per block on all of them (mchip_mfma16_fast_grid picks the count). Every C
 // element gets the same MFMA sequence either way, so the results are the
 // same bits.
-template <bool kBf16, bool kPackedA, typename Epilogue>
-__device__ __forceinline__ void mc_gemm16_fast(const unsigned short* __restrict__ a, const unsigned short* __restrict__ b,
-                                               float* __restrict__ c, int m, int n, int k, const Epilogue& epilogue) {
+template <bool kBf16, bool kPackedA, bool kPackedB, typename Epilogue>
+__device__ __forceinline__ void mc_gemm16_tiles(const unsigned short* __restrict__ a, const unsigned short* __restrict__ b,
+                                                float* __restrict__ c, int m, int n, int k, const Epilogue& epilogue) {
     __shared__ __attribute__((aligned(1024))) unsigned char smem[kFStages * kFStage];
     MC_LDS unsigned char* lds = (MC_LDS unsigned char*)(smem);  // generic -> LDS address space
 
@@ -400,7 +432,7 @@ __device__ __forceinline__ void mc_gemm16_fast(const unsigned short* __restrict_
     const int bid = static_cast<int>(blockIdx.x);
     if (bid < full) {
         const int tm = bid / tiles_n, tn = bid % tiles_n;
-        fast_tile<kBf16, kFBM, kPackedA>(lds, a, b, c, m, n, k, tm * kFBM, tn * kFBN, epilogue);
+        fast_tile<kBf16, kFBM, kPackedA, kPackedB>(lds, a, b, c, m, n, k, tm * kFBM, tn * kFBN, epilogue);
     } else {
         const int t = full + (bid - full) / 2, half = (bid - full) % 2;
         const int tm = t / tiles_n, tn = t % tiles_n;
@@ -409,6 +441,21 @@ __device__ __forceinline__ void mc_gemm16_fast(const unsigned short* __restrict_
         // of C: it has nothing to store, and its clamped rows would sit
         // before its origin (fetch offsets below zero).
         if (row0 >= m) return;
-        fast_tile<kBf16, kFBM / 2, kPackedA>(lds, a, b, c, m, n, k, row0, tn * kFBN, epilogue);
+        fast_tile<kBf16, kFBM / 2, kPackedA, kPackedB>(lds, a, b, c, m, n, k, row0, tn * kFBN, epilogue);
     }
+}
+
+// Row-major B (and A row-major or packed).
+template <bool kBf16, bool kPackedA, typename Epilogue>
+__device__ __forceinline__ void mc_gemm16_fast(const unsigned short* __restrict__ a, const unsigned short* __restrict__ b,
+                                               float* __restrict__ c, int m, int n, int k, const Epilogue& epilogue) {
+    mc_gemm16_tiles<kBf16, kPackedA, false>(a, b, c, m, n, k, epilogue);
+}
+
+// Both operands packed, K the padded one (a multiple of 64); any M and N.
+template <bool kBf16, typename Epilogue>
+__device__ __forceinline__ void mc_gemm16_packed(const unsigned short* __restrict__ a,
+                                                 const unsigned short* __restrict__ b, float* __restrict__ c, int m,
+                                                 int n, int k, const Epilogue& epilogue) {
+    mc_gemm16_tiles<kBf16, true, true>(a, b, c, m, n, k, epilogue);
 }

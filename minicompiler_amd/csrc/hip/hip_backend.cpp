@@ -35,10 +35,10 @@ constexpr std::size_t kArenaAlign = 256;
 
 std::size_t align_up(std::size_t v) { return (v + kArenaAlign - 1) / kArenaAlign * kArenaAlign; }
 
-// Bytes of a converted tensor-core matmul's packed A (its workspace's first part).
-template <class L>
-std::size_t packed_a_bytes(const L& l) {
-    return align_up(static_cast<std::size_t>(mchip_packed_a16_elements(l.m, l.k)) * 2);
+// Bytes of a packed operand of `rows` rows (columns) of a converted
+// tensor-core matmul: packed A, then packed B, make up its workspace.
+std::size_t packed_bytes(int rows, int k) {
+    return align_up(static_cast<std::size_t>(mchip_packed_a16_elements(rows, mchip_pack16_k(k))) * 2);
 }
 
 Status hip_status(int rc, const char* call) {
@@ -100,10 +100,13 @@ struct Launch {
     std::vector<void*> sum_params;
     // Tensor-core matmul on fp32 operands rounded to 16 bits in the launch's
     // workspace (a16, b16) first: per run, or once at compile time for a
-    // constant operand. a16 holds A packed (mchip_convert_pack_a_f32: 256-row
-    // bands of 16 KiB K-step blocks in the kernel's LDS order), b16 B row-major.
+    // constant operand. Both are packed (mchip_pack16_a_f32, mchip_pack16_b_f32:
+    // 256-row bands and 256-column panels of 16 KiB K-step blocks in the
+    // kernels' fragment order, K padded with zeros to kp).
     bool lowp = false;
     int dtype = 0;
+    int kp = 0;
+    int frag = MCHIP_FRAG_NONE;  // the small-tile shape, or the 256x256 tiles
     void* a16 = nullptr;
     void* b16 = nullptr;
     bool convert_a = false, convert_b = false;
@@ -195,7 +198,7 @@ public:
                     l.body = fused_body(l);
                 }
                 const std::size_t ws =
-                    l.lowp ? packed_a_bytes(l) + align_up(static_cast<std::size_t>(l.k) * l.n * 2)
+                    l.lowp ? packed_bytes(l.m, l.k) + packed_bytes(l.n, l.k)
                            : matmul_workspace_bytes(l.matmul, l.m, l.n, l.splits);
                 workspace_offset.push_back(ws ? top : SIZE_MAX);
                 if (ws) top += align_up(ws);
@@ -219,7 +222,7 @@ public:
             Launch& l = launches_[j];
             if (l.lowp) {
                 l.a16 = base + workspace_offset[j];
-                l.b16 = base + workspace_offset[j] + packed_a_bytes(l);
+                l.b16 = base + workspace_offset[j] + packed_bytes(l.m, l.k);
             } else {
                 l.workspace = reinterpret_cast<float*>(base + workspace_offset[j]);
             }
@@ -238,14 +241,8 @@ public:
         // Constant operands of converted tensor-core matmuls: rounded once, here.
         for (const Launch& l : launches_) {
             if (!l.lowp) continue;
-            if (!l.convert_a) {
-                MCHIP_TRY(mchip_convert_pack_a_f32(l.dtype, static_cast<const float*>(value_ptr(a_of(l))), l.a16, l.m,
-                                                   l.k, stream_));
-            }
-            if (!l.convert_b) {
-                MCHIP_TRY(mchip_convert_f32(l.dtype, static_cast<const float*>(value_ptr(b_of(l))), l.b16,
-                                            static_cast<std::size_t>(l.k) * l.n, stream_));
-            }
+            if (!l.convert_a) MCHIP_TRY(pack_a(l, stream_));
+            if (!l.convert_b) MCHIP_TRY(pack_b(l, stream_));
         }
         MCHIP_TRY(mchip_stream_synchronize(stream_));
 
@@ -490,23 +487,17 @@ private:
         }
         if (l.lowp) {
             int rc = 0;
-            if (l.convert_a) {
-                rc = mchip_convert_pack_a_f32(l.dtype, static_cast<const float*>(value_ptr(a_of(l))), l.a16, l.m, l.k,
-                                              s);
-            }
-            if (rc == 0 && l.convert_b) {
-                rc = mchip_convert_f32(l.dtype, static_cast<const float*>(value_ptr(b_of(l))), l.b16,
-                                       static_cast<std::size_t>(l.k) * l.n, s);
-            }
-            if (rc != 0) return hip_status(rc, "convert_f32");
+            if (l.convert_a) rc = pack_a(l, s);
+            if (rc == 0 && l.convert_b) rc = pack_b(l, s);
+            if (rc != 0) return hip_status(rc, "pack16");
             if (l.kind == Launch::Kind::FusedMatmul) {
-                rc = mchip_module_launch(l.function, l.grid_x, 512, 0, s, l.params.data());
+                rc = mchip_module_launch(l.function, l.grid_x, l.block, 0, s, l.params.data());
                 return rc == 0 ? Status() : hip_status(rc, "hipModuleLaunchKernel(mc_gemm_epilogue)");
             }
-            rc = mchip_launch_matmul_lowp_packed(static_cast<int>(l.matmul), l.dtype, l.a16, l.b16,
-                                                 static_cast<float*>(value_ptr(l.node)), l.m, l.n, l.k, s);
+            rc = mchip_launch_mfma16_packed(l.dtype, l.frag, l.a16, l.b16, static_cast<float*>(value_ptr(l.node)), l.m,
+                                            l.n, l.k, s);
             if (rc != 0) {
-                return Error{std::string("launch_matmul_lowp_packed(") + matmul_kernel_name(l.matmul) + "): " +
+                return Error{std::string("launch_mfma16_packed(") + matmul_kernel_name(l.matmul) + "): " +
                              mchip_error_string(rc)};
             }
             return Status();
@@ -534,6 +525,13 @@ private:
             return Error{std::string("launch_matmul(") + matmul_kernel_name(l.matmul) + "): " + mchip_error_string(rc)};
         }
         return Status();
+    }
+
+    int pack_a(const Launch& l, void* s) const {
+        return mchip_pack16_a_f32(l.dtype, static_cast<const float*>(value_ptr(a_of(l))), l.a16, l.m, l.k, s);
+    }
+    int pack_b(const Launch& l, void* s) const {
+        return mchip_pack16_b_f32(l.dtype, static_cast<const float*>(value_ptr(b_of(l))), l.b16, l.k, l.n, s);
     }
 
     // Whether the launch adds its K splits' partials itself (no sum launch),
@@ -615,12 +613,19 @@ private:
             l->matmul = l->splits > 1 ? MatmulKernel::SplitK : MatmulKernel::DoubleBuffered;
         }
         const bool bf16 = l->matmul == MatmulKernel::TensorCoreBf16, f16 = l->matmul == MatmulKernel::TensorCoreF16;
-        if (options_.convert_tensor_core_operands && (bf16 || f16) && mchip_mfma16_fast_fits(l->m, l->n, l->k)) {
+        const bool constant_b = graph_.node(node.inputs[1]).op == OpKind::Constant;
+        if (options_.convert_tensor_core_operands && (bf16 || f16) && mchip_pack16_fits(l->m, l->n, l->k) &&
+            (constant_b || mchip_mfma16_fast_fits(l->m, l->n, l->k))) {
             l->lowp = true;
             l->splits = 1;
             l->dtype = bf16 ? MCHIP_DTYPE_BF16 : MCHIP_DTYPE_F16;
+            l->kp = mchip_pack16_k(l->k);
+            // The small tiles split K over a block's waves; with B computed or
+            // fed per run the product keeps the operator's order of adds (the
+            // same bits as mchip_launch_tensor_core on the fp32 operands).
+            if (constant_b) l->frag = mchip_mfma16_packed_plan(l->m, l->n, device_.cu_count);
             l->convert_a = graph_.node(node.inputs[0]).op != OpKind::Constant;
-            l->convert_b = graph_.node(node.inputs[1]).op != OpKind::Constant;
+            l->convert_b = !constant_b;
         }
         return Status();
     }
@@ -629,7 +634,11 @@ private:
     // for the same kernel (operands in the arena or bound by the caller are
     // 16-byte aligned).
     GemmBody fused_body(Launch& l) const {
-        if (l.lowp) return l.dtype == MCHIP_DTYPE_BF16 ? GemmBody::Bf16Fast : GemmBody::F16Fast;
+        if (l.lowp) {
+            const bool bf16 = l.dtype == MCHIP_DTYPE_BF16;
+            if (l.frag != MCHIP_FRAG_NONE) return bf16 ? GemmBody::Bf16Frag : GemmBody::F16Frag;
+            return bf16 ? GemmBody::Bf16Packed : GemmBody::F16Packed;
+        }
         if (l.matmul == MatmulKernel::SplitK &&
             (l.ring_cfg == MCHIP_RING_NONE || l.ring_cfg == MCHIP_RING_NARROW)) {
             int shape = 0, splits = 0, k_split = 0;
@@ -738,7 +747,8 @@ private:
                 GemmDims dims;
                 dims.m = l.m;
                 dims.n = l.n;
-                dims.k = l.k;
+                dims.k = l.lowp ? l.kp : l.k;
+                dims.frag = l.frag;
                 dims.k_split = l.k_split;
                 dims.depth = l.depth;
                 k.source = generate_gemm_epilogue_kernel(*f.fused, acc, shapes, f.type.shape, l.n % 4 == 0 && l.k % 4 == 0,
@@ -783,7 +793,9 @@ private:
             sources_.push_back(kern.source);
             if (l.kind == Launch::Kind::FusedMatmul && l.lowp) {
                 l.function = built[j]->function;
-                l.grid_x = mchip_mfma16_fast_grid(l.m, l.n, device_.cu_count);
+                const bool frag = l.frag != MCHIP_FRAG_NONE;
+                l.grid_x = frag ? mchip_frag_grid(l.frag, l.m, l.n) : mchip_mfma16_fast_grid(l.m, l.n, device_.cu_count);
+                l.block = frag ? static_cast<unsigned>(mchip_frag_threads(l.frag)) : 512u;
                 l.grid_y = l.grid_z = 1;
                 l.epilogue_inputs.assign(graph_.node(l.epilogue_node).inputs.size(), nullptr);
                 continue;
@@ -842,7 +854,7 @@ private:
         // Stable argument addresses: the launch list no longer changes.
         for (Launch& l : launches_) {
             if (l.kind == Launch::Kind::FusedMatmul && l.lowp) {
-                l.params = {&l.a16, &l.b16, &l.c_ptr, &l.m, &l.n, &l.k, l.epilogue_inputs.data()};
+                l.params = {&l.a16, &l.b16, &l.c_ptr, &l.m, &l.n, &l.kp, l.epilogue_inputs.data()};
                 continue;
             }
             if (l.kind == Launch::Kind::FusedMatmul) {

@@ -38,6 +38,40 @@ int mchip_convert_pack_a_f32(int dtype, const float* a, void* packed, int m, int
 int mchip_launch_matmul_lowp_packed(int kernel, int dtype, const void* a_packed, const void* b, float* c, int m, int n,
                                     int k, void* stream);
 
+/* Both operands of a bf16/fp16 product packed from fp32, of any m, n, k
+ * (gemm_mfma16_fast.h: A in 256-row bands, B in 256-column panels, K padded
+ * with zeros to mchip_pack16_k(k)); a packed operand of r rows (columns)
+ * takes mchip_packed_a16_elements(r, mchip_pack16_k(k)) elements. Rows and
+ * columns of the last band past the operand are left as they are.
+ * mchip_pack16_fits: the sizes the kernels' 31-bit offsets allow.
+ * mchip_launch_mfma16_packed: the product, on 256x256 tiles
+ * (MCHIP_FRAG_NONE) or on the small tiles of gemm_mfma16_frag.h;
+ * mchip_mfma16_packed_plan picks between them, mchip_frag_* describe a
+ * small tile's launch. */
+enum {
+    MCHIP_FRAG_NONE = -1,
+    MCHIP_FRAG_16X16 = 0,
+    MCHIP_FRAG_16X32 = 1,
+    MCHIP_FRAG_16X64 = 2,
+    MCHIP_FRAG_32X16 = 3,
+    MCHIP_FRAG_32X32 = 4,
+    MCHIP_FRAG_32X64 = 5,
+    MCHIP_FRAG_64X16 = 6,
+    MCHIP_FRAG_64X32 = 7,
+    MCHIP_FRAG_64X64 = 8
+};
+int mchip_pack16_k(int k);
+int mchip_pack16_fits(int m, int n, int k);
+int mchip_pack16_a_f32(int dtype, const float* a, void* packed, int m, int k, void* stream);
+int mchip_pack16_b_f32(int dtype, const float* b, void* packed, int k, int n, void* stream);
+int mchip_mfma16_packed_plan(int m, int n, int cu_count);
+int mchip_frag_rows(int shape);
+int mchip_frag_cols(int shape);
+int mchip_frag_threads(int shape);
+unsigned mchip_frag_grid(int shape, int m, int n);
+int mchip_launch_mfma16_packed(int dtype, int shape, const void* a_packed, const void* b_packed, float* c, int m,
+                               int n, int k, void* stream);
+
 /* C = sum over z of partial[z * count + i], added in z order. */
 int mchip_sum_split_partials(const float* partial, float* c, size_t count, int splits, void* stream);
 

@@ -19,5 +19,8 @@ extern const char* const kGemmSplitArrivalSource;
 // gemm_mfma16_fast.h: the bf16 / fp16 matrix-core GEMM body (16-bit inputs
 // in HBM) with an epilogue hook.
 extern const char* const kGemm16FastSource;
+// gemm_mfma16_frag.h: the small-tile body on packed 16-bit operands (goes
+// after kGemm16FastSource).
+extern const char* const kGemm16FragSource;
 
 }  // namespace minicompiler::hip
