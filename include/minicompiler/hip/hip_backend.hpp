@@ -76,13 +76,15 @@ struct HipOptions {
     // the store of an FP32 matrix-core GEMM (one kernel instead of two), when
     // the memory plan makes that safe.
     bool fuse_epilogue = true;
-    // Tensor-core matmuls (bf16 / fp16) in a compiled graph: round the fp32
-    // operands to 16 bits into workspace first (constants once, at compile
-    // time), then run the 256x256-tile kernel on them, when the shape allows
-    // (K a multiple of 64, N a multiple of 8). The rounding and the
-    // accumulation order are those of the staging kernel with K unsplit, so
-    // results match that kernel bit for bit. Off: the staging kernel rounds
-    // while it stages (and splits K where SplitK would).
+    // Tensor-core matmuls (bf16 / fp16) in a compiled graph: round and pack
+    // the fp32 operands to 16 bits in workspace first (constants once, at
+    // compile time), then run the packed kernels on them: any shape with a
+    // constant B; with a B computed or fed per run, K a multiple of 64 and N
+    // of 8. On the 256x256 tiles the rounding and the accumulation order are
+    // those of the operator's kernel with K unsplit (the same bits); the
+    // small tiles for products that would leave the chip idle (constant B
+    // only) split K over a block's waves. Off: the operator's kernel rounds
+    // while it loads (and splits K where SplitK would).
     bool convert_tensor_core_operands = true;
     // enqueue() captures its launches into a HIP graph the first time and
     // replays that graph afterwards (one submission instead of one per

@@ -171,7 +171,7 @@ int mchip_launch_matmul_cfg(int kernel, const float* a, const float* b, float* c
  * 1 for kernels that do not split; 0 for invalid sizes or a configuration
  * that cannot run the product. */
 int mchip_matmul_k_ranges(int kernel, int m, int n, int k, int splits, int ring_cfg);
-int mchip_tensor_core_k_ranges(int k, int splits);
+int mchip_tensor_core_k_ranges(int m, int n, int k, int splits);
 
 /* mchip_launch_matmul_cfg for split_k that adds the K splits' partials in
  * the GEMM launch itself where the ring or narrow body runs the product: the

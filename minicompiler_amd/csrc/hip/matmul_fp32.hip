@@ -634,7 +634,7 @@ extern "C" int mchip_matmul_k_ranges(int kernel, int m, int n, int k, int splits
             return p.status == hipSuccess ? p.depth : 0;
         }
         case kTensorCoreBf16:
-        case kTensorCoreF16: return mchip_tensor_core_k_ranges(k, splits);
+        case kTensorCoreF16: return mchip_tensor_core_k_ranges(m, n, k, splits);
         default: return 1;
     }
 }

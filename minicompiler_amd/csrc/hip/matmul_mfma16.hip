@@ -7,16 +7,22 @@
 // TF32 does not exist on gfx950 (no xf32 matrix instruction): those requests
 // report hipErrorNotSupported.
 //
-// Block tile 128x128, K step 64, 256 lanes = 4 waves in a 2x2 grid, each wave
-// a 64x64 quadrant as 4x4 16x16 accumulators. A is staged row-major
-// (k contiguous), B transposed (n-major, k contiguous), so each lane's MFMA
-// operand is one 16-byte LDS read. Two LDS stages; split-K as in the FP32
-// kernels.
+// The kernels:
+//   matmul_mfma16_staged   row-major operands, fp32 (rounded on the way into
+//                          LDS) or 16-bit, any shape and alignment, split K;
+//   matmul_mfma16_fast     16-bit operands, B row-major, 256x256 tiles
+//                          (gemm_mfma16_fast.h);
+//   matmul_mfma16_packed, matmul_mfma16_frag   both operands packed
+//                          (gemm_mfma16_fast.h, gemm_mfma16_frag.h).
+// Every kernel that does not split K adds each element's products in the same
+// order (32 k per MFMA, K ascending), so they give the same bits, except the
+// frag kernels, which split K over a block's waves.
 //
 // v_mfma_f32_16x16x32_*: lane l supplies row (A) / column (B) l % 16 and
 // eight k values from group l / 16; A and B use the same k assignment, so
 // any assignment gives the same sum (here group g holds k = 8g .. 8g+7 of the
-// 32-wide step). Result: value v of lane l is row 4 (l / 16) + v, column l % 16.
+// 32-wide step). Issued with B first the result is transposed: value v of
+// lane l is row l % 16, column 4 (l / 16) + v.
 
 #include "matmul.h"
 
@@ -62,143 +68,336 @@ __device__ __forceinline__ unsigned short to_bits(float x) {
     return to_f16_bits(x);
 }
 
+// Eight floats rounded to 16 bits (to nearest even), as the 16-byte chunk of
+// an MFMA operand. bf16: the hardware's packed conversion, the same bits as
+// to_bf16_bits (checked over all exponents, subnormals, infinities and NaNs).
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+typedef unsigned short u16x8u __attribute__((ext_vector_type(8), aligned(2)));
+typedef unsigned short u16x4u __attribute__((ext_vector_type(4), aligned(2)));
+typedef unsigned short u16x2u __attribute__((ext_vector_type(2), aligned(2)));
+typedef float f32x8 __attribute__((ext_vector_type(8)));
+
 template <bool kBf16>
-__device__ __forceinline__ f32x4 mfma(u16x8 a, u16x8 b, f32x4 c) {
-    if constexpr (kBf16) {
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b),
-                                                       c, 0, 0, 0);
-    } else {
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c,
-                                                      0, 0, 0);
-    }
+__device__ __forceinline__ u16x8 round8(f32x8 v) {
+    if constexpr (kBf16) return __builtin_bit_cast(u16x8, __builtin_convertvector(v, bf16x8));
+    return __builtin_bit_cast(u16x8, __builtin_convertvector(v, f16x8));
 }
 
-constexpr int kBM = 128, kBN = 128, kBK = 64;
-constexpr int kPitch = kBK + 8;  // halves per LDS row: 144 bytes, keeps 16-byte alignment
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 
-// Element source: fp32 in memory (rounded here) or 16-bit already.
-template <bool kBf16, bool kF32In>
-struct Source {
-    using T = typename std::conditional<kF32In, float, unsigned short>::type;
+template <bool kBf16>
+__device__ __forceinline__ u16x4 round4(f32x4 v) {
+    if constexpr (kBf16) return __builtin_bit_cast(u16x4, __builtin_convertvector(v, bf16x4));
+    return __builtin_bit_cast(u16x4, __builtin_convertvector(v, f16x4));
+}
+
+// ---------------------------------------------------------------- staged
+//
+// Row-major A [m, k] and B [k, n] of fp32 or 16-bit elements at any element
+// address. What bounds it: at fp32 operands the CU's vector-memory path (a
+// 128x128x64 step loads 64 KiB for 512 cycles of MFMA); at small products the
+// latency of each step's loads.
+//
+// Block tile kBM x kBN, K step 64, 256 lanes = 4 waves. A step's operands are
+// loaded into registers one step ahead, rounded there (fp32), and written to
+// one of two LDS stages in the fragment order of the packed layouts: per 32 k,
+// 1 KiB per 16 rows (columns), the 16-byte chunk of 8 k of row r, chunk c at
+// 256 c + 16 (r % 16 ^ swizzle). So each MFMA operand is one linear,
+// conflict-free ds_read_b128. A lane loads 8 k of a row of A per chunk; of B
+// it loads 8 k rows of kCV neighbouring columns and transposes them in
+// registers (the fp32 form by choosing which two floats each packed conversion
+// takes), where the form before this one wrote B to LDS two bytes at a time.
+// The swizzles (chunk of 64 k for A; column block for B) spread 8 consecutive
+// lanes' 16-byte writes over all banks.
+//
+// The edges. Rows past m read row m - 1. A lane whose columns cross n reads
+// the last kCV columns instead and writes them to those columns' places (a
+// neighbour writes the same values there), so no load is guarded; what lies
+// past n in LDS is never stored from. The last K step, when it is not whole,
+// is loaded element by element with zeros past K, as is everything when
+// n < kCV. Vector loads need element alignment only.
+//
+// On an MI355X, graph-timed, against the 128x128 kernel this one replaced:
+// 2048^3 fp32 operands as bf16 283.5 -> 42.7 us, 4096^3 1087 -> 242, 1000^3
+// (4 splits allowed) 45.2 -> 15.3; bf16 operands 1000^3 26.5 -> 12.0,
+// 3000x3001x1023 351 -> 58, 16x4096x4096 29.0 -> 11.2.
+// kWM x kWN waves of a group tile the block's C tile; kG groups take every
+// kG-th K step each and are added at the end; kAhead: steps loaded ahead (in
+// registers); kBlocks: blocks per CU the register budget is cut for; kAcc: 1,
+// or 4 accumulators per element that take the 32-wide half steps in turn and
+// are added at the end. Where a caller allows K ranges, the 128x128 kernel ran
+// up to four times the ranges these smaller tiles need to fill the chip; four
+// accumulators keep its number of partial sums, and so its rounding error.
+template <int kBM_, int kBN_, int kWM_, int kWN_, int kG_, int kAhead_, int kBlocks_, int kAcc_ = 1>
+struct Staged {
+    static constexpr int kBM = kBM_, kBN = kBN_, kBK = 64;
+    static constexpr int kG = kG_, kAhead = kAhead_, kBlocks = kBlocks_, kAcc = kAcc_;
+    static_assert(kAhead == 1 || kAhead == 2, "the main loop's unrolling");
+    static_assert(kAcc == 1 || (kAcc == 4 && kAhead == 2), "step parities known to the unrolled loop");
+    static constexpr int kWavesN = kWN_, kWaves = kWM_ * kWN_;
+    static constexpr int kLanes = 64 * kWaves, kThreads = kLanes * kG;
+    static constexpr int kRows = kBM / kWM_, kCols = kBN / kWN_;  // of a wave
+    static constexpr int kRowFrags = kRows / 16, kColFrags = kCols / 16;
+    // 16-byte loads of A per lane and step: 8 16-bit or 4 fp32 elements.
+    static constexpr int a_loads(bool f32) { return kBM * (f32 ? 16 : 8) / kLanes; }
+    static constexpr int kCV = kBN * 8 / kLanes;       // columns of B per lane
+    static constexpr int kASub = kBM * 64, kBSub = kBN * 64;  // bytes per 32 k
+    static constexpr int kStage = 2 * (kASub + kBSub);
+    static constexpr int kStagePitch = kStage + 1024;  // and 16 bytes per lane for columns before the tile
+    static constexpr int kSums = kG > 1 ? kG * kBM * kBN * 4 : 0;
+    static constexpr int kLds = kSums > 2 * kStagePitch * kG ? kSums : 2 * kStagePitch * kG;
 };
 
-// Four consecutive elements as 16-bit patterns; zeros out of range.
-template <bool kBf16, bool kF32In, bool kVec>
-__device__ __forceinline__ u16x4 load4(const void* __restrict__ base, int row, int col, int row_end, int col_end,
-                                       int ld) {
-    u16x4 v = {0, 0, 0, 0};
-    if (row >= row_end) return v;
-    if constexpr (kF32In) {
-        const float* s = static_cast<const float*>(base) + static_cast<std::ptrdiff_t>(row) * ld + col;
-        if constexpr (kVec) {
-            if (col < col_end) {
-                const f32x4 f = *reinterpret_cast<const f32x4*>(s);
-                v = u16x4{to_bits<kBf16>(f.x), to_bits<kBf16>(f.y), to_bits<kBf16>(f.z), to_bits<kBf16>(f.w)};
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if (col + e < col_end) v[e] = to_bits<kBf16>(s[e]);
-            }
-        }
-    } else {
-        const unsigned short* s =
-            static_cast<const unsigned short*>(base) + static_cast<std::ptrdiff_t>(row) * ld + col;
-        if constexpr (kVec) {
-            if (col < col_end) v = *reinterpret_cast<const u16x4*>(s);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                if (col + e < col_end) v[e] = s[e];
-            }
-        }
-    }
-    return v;
-}
+// A K step's parity, as a type.
+template <int kParity>
+struct Parity {
+    static constexpr int value = kParity;
+};
 
-template <bool kBf16, bool kF32In, bool kVec>
-__global__ void __launch_bounds__(256, 2) matmul_mfma16(const void* __restrict__ a, const void* __restrict__ b,
-                                                        float* __restrict__ c, int m, int n, int k, int k_split,
-                                                        float* __restrict__ partial) {
-    __shared__ __attribute__((aligned(16))) unsigned short as[2][kBM][kPitch];
-    __shared__ __attribute__((aligned(16))) unsigned short bt[2][kBN][kPitch];
+// kCV consecutive elements as 16-byte aligned or unaligned vector loads.
+template <bool kF32In, int kCV>
+struct BVec;
+template <>
+struct BVec<true, 4> { typedef f32x4u type; };
+template <>
+struct BVec<true, 2> { typedef f32x2u type; };
+template <>
+struct BVec<false, 4> { typedef u16x4u type; };
+template <>
+struct BVec<false, 2> { typedef u16x2u type; };
 
-    const int tid = threadIdx.x;
+template <bool kBf16, bool kF32In, class Cfg>
+__global__ void __launch_bounds__(Cfg::kThreads, Cfg::kBlocks) matmul_mfma16_staged(const void* __restrict__ a_, const void* __restrict__ b_,
+                                                               float* __restrict__ c, int m, int n, int k, int k_split,
+                                                               float* __restrict__ partial) {
+    typedef typename std::conditional<kF32In, float, unsigned short>::type T;
+    typedef typename BVec<kF32In, Cfg::kCV>::type BV;
+    constexpr int kCV = Cfg::kCV, kBK = Cfg::kBK;
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[Cfg::kLds];
+    const T* __restrict__ a = static_cast<const T*>(a_);
+    const T* __restrict__ b = static_cast<const T*>(b_);
+
+    const int grp = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / Cfg::kLanes);
+    const int tid = static_cast<int>(threadIdx.x) % Cfg::kLanes;  // in the group
     const int wave = tid / 64, lane = tid % 64;
-    const int wr = (wave / 2) * 64, wc = (wave % 2) * 64;
-    const int g = lane / 16, li = lane % 16;
-    const int row0 = blockIdx.y * kBM, col0 = blockIdx.x * kBN;
-    const int kb = blockIdx.z * k_split;
-    const int ke = min(k, kb + k_split);
+    unsigned char* const stages = smem + grp * 2 * Cfg::kStagePitch;
+    // Tiles in column groups of 8, row by row within a group; block L runs on
+    // XCD L % 8, which takes a contiguous eighth of the list when the count is
+    // a multiple of 8, so an L2 serves a compact patch of tiles.
+    const int tiles_n = (n + Cfg::kBN - 1) / Cfg::kBN, tiles_m = (m + Cfg::kBM - 1) / Cfg::kBM;
+    const int total = static_cast<int>(gridDim.x), L = static_cast<int>(blockIdx.x);
+    int q = total % 8 == 0 ? (L % 8) * (total / 8) + L / 8 : L;
+    const int z = q / (tiles_m * tiles_n);
+    q -= z * tiles_m * tiles_n;
+    const int group = q / (8 * tiles_m), in_group = q % (8 * tiles_m);
+    const int width = min(8, tiles_n - 8 * group);
+    const int row0 = (in_group / width) * Cfg::kBM, col0 = (8 * group + in_group % width) * Cfg::kBN;
+    const int kb = z * k_split, ke = min(k, kb + k_split);
 
-    f32x4 acc[4][4];
+    // This lane's loads of A, a row's 64 k over 8 (16) consecutive lanes:
+    // row tid / 8 (16) + .., k kAK ac .. kAK ac + kAK - 1 of the step.
+    constexpr int kALoads = Cfg::a_loads(kF32In), kAK = kF32In ? 4 : 8, kARow = kBK / kAK;
+    const int ac = tid % kARow;
+    const T* a_src[kALoads];
+    int a_dst[kALoads];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-
-    // A tile: 128 rows x 16 quads; B tile: 64 rows x 32 quads. 8 of each per lane.
-    u16x4 ra[8], rb[8];
-    auto global_load = [&](int k0) {
-#pragma unroll
-        for (int l = 0; l < 8; ++l) {
-            const int f = tid + l * 256;
-            ra[l] = load4<kBf16, kF32In, kVec>(a, row0 + f / 16, k0 + (f % 16) * 4, m, ke, k);
-            rb[l] = load4<kBf16, kF32In, kVec>(b, k0 + f / 32, col0 + (f % 32) * 4, ke, n, n);
-        }
-    };
-    auto lds_store = [&](int s) {
-#pragma unroll
-        for (int l = 0; l < 8; ++l) {
-            const int f = tid + l * 256;
-            *reinterpret_cast<u16x4*>(&as[s][f / 16][(f % 16) * 4]) = ra[l];
-            const int kk = f / 32, cc = (f % 32) * 4;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) bt[s][cc + e][kk] = rb[l][e];
-        }
-    };
-    auto multiply = [&](int s) {
-#pragma unroll
-        for (int q = 0; q < kBK / 32; ++q) {
-            u16x8 av[4], bv[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) av[i] = *reinterpret_cast<const u16x8*>(&as[s][wr + i * 16 + li][q * 32 + g * 8]);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) bv[j] = *reinterpret_cast<const u16x8*>(&bt[s][wc + j * 16 + li][q * 32 + g * 8]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = mfma<kBf16>(av[i], bv[j], acc[i][j]);
-        }
-    };
-
-    const int tiles = ke > kb ? (ke - kb + kBK - 1) / kBK : 0;
-    if (tiles > 0) {
-        global_load(kb);
-        lds_store(0);
+    for (int i = 0; i < kALoads; ++i) {
+        const int r = tid / kARow + Cfg::kLanes / kARow * i;
+        const int ch = ac * kAK / 8;  // its chunk of 8 k
+        a_src[i] = a + static_cast<std::ptrdiff_t>(min(row0 + r, m - 1)) * k + kAK * ac;
+        a_dst[i] = (ch / 4) * Cfg::kASub + (r / 16) * 1024 + (ch % 4) * 256 + ((r % 16) ^ ch) * 16 +
+                   (kF32In ? (ac % 2) * 8 : 0);
     }
-    __syncthreads();
-    for (int t = 0; t < tiles; ++t) {
-        const int cur = t & 1;
-        const bool more = t + 1 < tiles;
-        if (more) global_load(kb + (t + 1) * kBK);
-        multiply(cur);
-        if (more) lds_store(cur ^ 1);
+    // This lane's columns of B: bcol .. bcol + kCV - 1, k 8 bk .. 8 bk + 7.
+    const bool whole_cols = n >= kCV;
+    constexpr int kQuads = Cfg::kBN / kCV;
+    const int bk = tid / kQuads;
+    const int bcol = whole_cols ? min(col0 + (tid % kQuads) * kCV, n - kCV) : (tid % kQuads) * kCV;
+    const T* const b_src = b + static_cast<std::ptrdiff_t>(8 * bk) * n + bcol;
+    int b_dst[kCV];
+#pragma unroll
+    for (int j = 0; j < kCV; ++j) {
+        const int col = bcol - col0 + j;  // may be before the tile: written past the stage
+        b_dst[j] = col < 0 ? Cfg::kStage + lane * 16
+                           : 2 * Cfg::kASub + (bk / 4) * Cfg::kBSub + (col / 16) * 1024 + (bk % 4) * 256 +
+                                 ((col % 16) ^ ((col / 16) & 3)) * 16;
+    }
+
+    typedef typename std::conditional<kF32In, f32x4u, u16x8u>::type AV;
+    struct Regs {
+        AV a[kALoads];
+        BV b[8];
+    };
+    auto load_whole = [&](Regs& r, int k0) {
+#pragma unroll
+        for (int i = 0; i < kALoads; ++i) r.a[i] = *reinterpret_cast<const AV*>(a_src[i] + k0);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            r.b[e] = *reinterpret_cast<const BV*>(b_src + static_cast<std::ptrdiff_t>(k0 + e) * n);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto load_part = [&](Regs& r, int k0) {
+#pragma unroll
+        for (int i = 0; i < kALoads; ++i)
+#pragma unroll
+            for (int e = 0; e < kAK; ++e) r.a[i][e] = k0 + kAK * ac + e < ke ? a_src[i][k0 + e] : T(0);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+#pragma unroll
+            for (int j = 0; j < kCV; ++j)
+                r.b[e][j] = k0 + 8 * bk + e < ke && bcol + j < n ? b_src[static_cast<std::ptrdiff_t>(k0 + e) * n + j] : T(0);
+    };
+    auto store = [&](const Regs& r, int stage) {
+        unsigned char* const s = stages + stage * Cfg::kStagePitch;
+#pragma unroll
+        for (int i = 0; i < kALoads; ++i) {
+            if constexpr (kF32In) {
+                *reinterpret_cast<u16x4*>(s + a_dst[i]) = round4<kBf16>(r.a[i]);
+            } else {
+                *reinterpret_cast<u16x8*>(s + a_dst[i]) = r.a[i];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < kCV; ++j) {
+            u16x8 v;
+            if constexpr (kF32In) {
+                v = round8<kBf16>(f32x8{r.b[0][j], r.b[1][j], r.b[2][j], r.b[3][j], r.b[4][j], r.b[5][j], r.b[6][j], r.b[7][j]});
+            } else {
+                v = u16x8{r.b[0][j], r.b[1][j], r.b[2][j], r.b[3][j], r.b[4][j], r.b[5][j], r.b[6][j], r.b[7][j]};
+            }
+            *reinterpret_cast<u16x8*>(s + b_dst[j]) = v;
+        }
+    };
+
+    const int wr = (wave / Cfg::kWavesN) * Cfg::kRows, wc = (wave % Cfg::kWavesN) * Cfg::kCols;
+    const int lk = lane / 16, li = lane % 16;
+    f32x4 sum[Cfg::kAcc][Cfg::kRowFrags][Cfg::kColFrags];
+#pragma unroll
+    for (int x = 0; x < Cfg::kAcc; ++x)
+#pragma unroll
+        for (int i = 0; i < Cfg::kRowFrags; ++i)
+#pragma unroll
+            for (int j = 0; j < Cfg::kColFrags; ++j) sum[x][i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto multiply = [&](int stage, auto parity) {
+        const unsigned char* const s = stages + stage * Cfg::kStagePitch;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            u16x8 av[Cfg::kRowFrags], bv[Cfg::kColFrags];
+#pragma unroll
+            for (int i = 0; i < Cfg::kRowFrags; ++i)
+                av[i] = *reinterpret_cast<const u16x8*>(s + h * Cfg::kASub + (wr / 16 + i) * 1024 + lk * 256 +
+                                                        (li ^ (4 * h + lk)) * 16);
+#pragma unroll
+            for (int j = 0; j < Cfg::kColFrags; ++j)
+                bv[j] = *reinterpret_cast<const u16x8*>(s + 2 * Cfg::kASub + h * Cfg::kBSub + (wc / 16 + j) * 1024 +
+                                                        lk * 256 + (li ^ ((wc / 16 + j) & 3)) * 16);
+#pragma unroll
+            for (int i = 0; i < Cfg::kRowFrags; ++i)
+#pragma unroll
+                for (int j = 0; j < Cfg::kColFrags; ++j) {
+                    f32x4& acc = sum[(2 * decltype(parity)::value + h) % Cfg::kAcc][i][j];
+                    acc = mc_mfma16<kBf16>(bv[j], av[i], acc);
+                }
+        }
+    };
+
+    // The group's i-th whole step is step i kG + grp, for i < mine: the same
+    // count for every group, so the barriers match. Register set i % kAhead
+    // holds it, loaded kAhead steps before it is written to LDS. Every load
+    // is unconditional (past the last it loads that one again): under a
+    // condition, the compiler's wait for one set would wait for the sets
+    // loaded after it too. What is left is at most one more step per group,
+    // whole, partial or empty (zeros), loaded ahead as well where there are
+    // registers for it; with n < kCV every step is of that kind.
+    constexpr int kAhead = Cfg::kAhead, kG = Cfg::kG;
+    const int tiles = ke > kb ? (ke - kb + kBK - 1) / kBK : 0;
+    const int full = whole_cols ? (ke - kb) / kBK : 0;
+    const int mine = full / kG;
+    const int rounds = (tiles + kG - 1) / kG;
+    constexpr bool kRestAhead = kAhead > 1;
+    auto k_of = [&](int i) { return kb + (i * kG + grp) * kBK; };
+    auto load_rest = [&](Regs& r, int i) {
+        if (i * kG + grp < full) {
+            load_whole(r, k_of(i));
+        } else {
+            load_part(r, k_of(i));
+        }
+    };
+    Regs rest;
+    if (mine > 0) {
+        Regs set[kAhead];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) load_whole(set[u], k_of(min(u, mine - 1)));
+        if (kRestAhead && mine < rounds) load_rest(rest, mine);
+        store(set[0], 0);
+        load_whole(set[0], k_of(min(kAhead, mine - 1)));
+        __syncthreads();
+        auto step = [&](int i, Regs& next, auto parity) {
+            // The other stage was last read before the previous barrier.
+            store(next, (i + 1) & 1);
+            load_whole(next, k_of(min(i + 1 + kAhead, mine - 1)));
+            multiply(i & 1, parity);
+            __syncthreads();
+        };
+        int i = 0;
+        for (; i + kAhead <= mine; i += kAhead) {
+            step(i, set[1 % kAhead], Parity<0>{});
+            if constexpr (kAhead == 2) step(i + 1, set[0], Parity<1>{});
+        }
+        if (i < mine) step(i, set[1 % kAhead], Parity<0>{});
+    }
+    for (int i = mine; i < rounds; ++i) {
+        if (!kRestAhead || mine == 0 || i > mine) load_rest(rest, i);
+        store(rest, i & 1);
+        __syncthreads();
+        multiply(i & 1, Parity<1>{});
         __syncthreads();
     }
 
-    float* __restrict__ out = gridDim.z == 1 ? c : partial + static_cast<std::ptrdiff_t>(blockIdx.z) * m * n;
+    f32x4(&acc)[Cfg::kRowFrags][Cfg::kColFrags] = sum[0];
+    if constexpr (Cfg::kAcc == 4) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < Cfg::kRowFrags; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int col = col0 + wc + j * 16 + li;
-            if (col >= n) continue;
+            for (int j = 0; j < Cfg::kColFrags; ++j) acc[i][j] = (sum[0][i][j] + sum[1][i][j]) + (sum[2][i][j] + sum[3][i][j]);
+    }
+    // Lane l holds row l % 16, columns 4 (l / 16) .. + 3 of each fragment.
+    float* __restrict__ out = partial != nullptr ? partial + static_cast<std::ptrdiff_t>(z) * m * n : c;
+    auto store_c = [&](int i, int j, f32x4 v) {
+        const int row = row0 + wr + i * 16 + li, col = col0 + wc + j * 16 + 4 * lk;
+        if (row >= m) return;
+        float* const dst = out + static_cast<std::ptrdiff_t>(row) * n + col;
+        if (col + 4 <= n) {
+            *reinterpret_cast<f32x4u*>(dst) = v;
+        } else {
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int row = row0 + wr + i * 16 + 4 * g + v;
-                if (row < m) out[static_cast<std::ptrdiff_t>(row) * n + col] = acc[i][j][v];
-            }
+            for (int e = 0; e < 3; ++e)
+                if (col + e < n) dst[e] = v[e];
+        }
+    };
+    if constexpr (kG == 1) {
+#pragma unroll
+        for (int i = 0; i < Cfg::kRowFrags; ++i)
+#pragma unroll
+            for (int j = 0; j < Cfg::kColFrags; ++j) store_c(i, j, acc[i][j]);
+    } else {
+        // The groups' tiles through LDS (the stages are done with), added in
+        // group order, every group a share of the fragments.
+        constexpr int kFrags = Cfg::kRowFrags * Cfg::kColFrags;
+        f32x4* const sums = reinterpret_cast<f32x4*>(smem);
+        auto at = [&](int g, int f) { return ((g * Cfg::kWaves + wave) * kFrags + f) * 64 + lane; };
+#pragma unroll
+        for (int f = 0; f < kFrags; ++f) sums[at(grp, f)] = acc[f / Cfg::kColFrags][f % Cfg::kColFrags];
+        __syncthreads();
+#pragma unroll
+        for (int f = 0; f < kFrags; ++f) {
+            if (f % kG != grp) continue;
+            f32x4 v = sums[at(0, f)];
+#pragma unroll
+            for (int g = 1; g < kG; ++g) v += sums[at(g, f)];
+            store_c(f / Cfg::kColFrags, f % Cfg::kColFrags, v);
         }
     }
 }
@@ -230,14 +429,6 @@ __global__ void __launch_bounds__(Cfg::kThreads) matmul_mfma16_frag(const unsign
     mc_gemm16_frag<kBf16, Cfg>(a, b, c, m, n, k, McGemm16Store{});
 }
 
-// The fast path takes 16-bit A and B with K a multiple of 64, N a multiple
-// of 8 (every 16-byte B chunk wholly inside or outside a row), A, B and C
-// 16-byte aligned, and no split.
-bool fast_eligible(const void* a, const void* b, const float* c, int m, int n, int k, int splits) {
-    const auto al = [](const void* p) { return reinterpret_cast<std::uintptr_t>(p) % 16 == 0; };
-    return splits <= 1 && mchip_mfma16_fast_fits(m, n, k) && al(a) && al(b) && al(c);
-}
-
 // CUs of the current device, asked once per device.
 int device_cus() {
     static std::atomic<int> cache[64];
@@ -251,6 +442,22 @@ int device_cus() {
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
     if (dev >= 0 && dev < 64) cache[dev].store(cus, std::memory_order_relaxed);
     return cus;
+}
+
+// Whether the 256x256-tile kernel can run the product: 16-bit A and B with K
+// a multiple of 64, N a multiple of 8 (every 16-byte B chunk wholly inside or
+// outside a row), A, B and C 16-byte aligned.
+bool fast_eligible(const void* a, const void* b, const float* c, int m, int n, int k) {
+    const auto al = [](const void* p) { return reinterpret_cast<std::uintptr_t>(p) % 16 == 0; };
+    return mchip_mfma16_fast_fits(m, n, k) && al(a) && al(b) && al(c);
+}
+
+// And whether it should, on row-major operands: with at most two 64x64 tiles
+// per CU the staged kernel is faster (bf16, K = 2048, graph-timed on an
+// MI355X: 512x1024 19.4 us against 30.8, 1024x2048 23.8 against 32.3, 1536x2048
+// 32.6 against 33.0; 2048^2 on its 128x128 tiles 34.7 against 34.4).
+bool fast_preferred(int m, int n) {
+    return static_cast<long long>((m + 63) / 64) * ((n + 63) / 64) > 2LL * std::max(device_cus(), 1);
 }
 
 template <bool kBf16, bool kPackedA = false>
@@ -314,8 +521,6 @@ __global__ void __launch_bounds__(256) pack_a16_kernel(const unsigned short* __r
 // took 22.1, and 512x4096 in 3.2 us against 8.7 (its regions were too few).
 // `blocks16` 16-row blocks are written, rows past m as zeros; a product reads
 // only those that hold a row (mchip_pack16_a_f32 writes no others).
-typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-
 template <bool kBf16>
 __global__ void __launch_bounds__(256) pack16_a_rows(const float* __restrict__ in, u32x4* __restrict__ out, int m,
                                                      int k, int kp, int pairs, long long units) {
@@ -324,15 +529,14 @@ __global__ void __launch_bounds__(256) pack16_a_rows(const float* __restrict__ i
     for (long long w = static_cast<long long>(blockIdx.x) * 4 + (threadIdx.x >> 6); w < units; w += waves) {
         const int rb = static_cast<int>(w / pairs), s0 = static_cast<int>(w % pairs) * 2;
         const int row = rb * 16 + (lane & 15);
-        float v[2][8];
+        f32x8 v[2];
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             const int kk = (s0 + u) * kFBK + (lane >> 4) * 8;
             const float* src = in + static_cast<long long>(row) * k + kk;
             if (row < m && kk + 8 <= k) {
                 const f32x4 lo = *reinterpret_cast<const f32x4u*>(src), hi = *reinterpret_cast<const f32x4u*>(src + 4);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[u][e] = lo[e], v[u][4 + e] = hi[e];
+                v[u] = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) v[u][e] = row < m && kk + e < k ? src[e] : 0.0f;
@@ -340,12 +544,8 @@ __global__ void __launch_bounds__(256) pack16_a_rows(const float* __restrict__ i
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-            u32x4 o;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                o[j] = to_bits<kBf16>(v[u][2 * j]) | (static_cast<unsigned>(to_bits<kBf16>(v[u][2 * j + 1])) << 16);
             const long long at = static_cast<long long>(rb / 16) * kp * 32 + (s0 + u) * 1024LL + (rb % 16) * 64 + lane;
-            out[at] = o;
+            out[at] = __builtin_bit_cast(u32x4, round8<kBf16>(v[u]));
         }
     }
 }
@@ -369,12 +569,9 @@ __global__ void __launch_bounds__(256) pack16_b(const float* __restrict__ in, u3
         for (int i = 0; i < kFBK; ++i) v[i] = k0 + i < k ? src[static_cast<long long>(i) * n] : 0.0f;
 #pragma unroll
         for (int ch = 0; ch < 4; ++ch) {
-            u32x4 o;
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                o[j] = to_bits<kBf16>(v[ch * 8 + 2 * j]) |
-                       (static_cast<unsigned>(to_bits<kBf16>(v[ch * 8 + 2 * j + 1])) << 16);
-            out[u * 1024 + (t >> 4) * 64 + ch * 16 + (t & 15)] = o;
+            const f32x8 w = {v[ch * 8],     v[ch * 8 + 1], v[ch * 8 + 2], v[ch * 8 + 3],
+                             v[ch * 8 + 4], v[ch * 8 + 5], v[ch * 8 + 6], v[ch * 8 + 7]};
+            out[u * 1024 + (t >> 4) * 64 + ch * 16 + (t & 15)] = __builtin_bit_cast(u32x4, round8<kBf16>(w));
         }
     }
 }
@@ -391,24 +588,96 @@ int split_len(int k, int splits, int step) {
     return (per + step - 1) / step * step;
 }
 
+// The staged kernel's tile and K ranges for a product (at most `splits`
+// ranges, what the caller sized its workspace for).
+struct StagedPlan {
+    int bm, bn, k_split, depth;
+    long long tiles;
+};
+
+// 128x128 tiles where they give at least four in five CUs one (the line of
+// split_k_splits, past which a caller has no workspace), else 64x64, or 32x64
+// for at most 32 rows; those in K ranges only where they leave half the CUs
+// idle (graph-timed on an MI355X, bf16 operands: 512x1024x2048, 128 tiles of
+// 64x64, 14.9 us in 2 ranges with their sum against 22.1 unsplit; 1000^3, 256
+// tiles, 12.5 us unsplit, where the 128x128 kernel in 4 ranges took 26.5).
+StagedPlan staged_plan(int m, int n, int k, int splits) {
+    const long long cus = std::max(device_cus(), 1);
+    const auto tiles = [&](int bm, int bn) {
+        return static_cast<long long>((m + bm - 1) / bm) * ((n + bn - 1) / bn);
+    };
+    StagedPlan p;
+    if (5 * tiles(128, 128) >= 4 * cus) {
+        p.bm = p.bn = 128;
+    } else {
+        p.bm = m <= 32 ? 32 : 64;
+        p.bn = 64;
+    }
+    p.tiles = tiles(p.bm, p.bn);
+    const long long want = std::max<long long>(1, std::min<long long>(splits, 2 * p.tiles <= cus ? cus / p.tiles : 1));
+    p.k_split = split_len(k, static_cast<int>(want), 64);
+    p.depth = std::max(1, (k + p.k_split - 1) / p.k_split);
+    return p;
+}
+
 template <bool kBf16, bool kF32In>
 int launch16(const void* a, const void* b, float* c, int m, int n, int k, hipStream_t stream, int splits,
              float* workspace) {
-    const int k_split = split_len(k, splits, kBK);
-    const int depth = std::max(1, (k + k_split - 1) / k_split);
-    if (depth > 1 && workspace == nullptr) return hipErrorInvalidValue;
-    const dim3 grid((n + kBN - 1) / kBN, (m + kBM - 1) / kBM, depth);
-    const std::uintptr_t align = kF32In ? 16 : 8;
-    const bool vec = n % 4 == 0 && k % 4 == 0 && aligned(a, align) && aligned(b, align);
-    float* ws = depth > 1 ? workspace : nullptr;
-    if (vec) {
-        hipLaunchKernelGGL((matmul_mfma16<kBf16, kF32In, true>), grid, dim3(256), 0, stream, a, b, c, m, n, k, k_split, ws);
+    // Several ranges asked for need a workspace, whatever number of them runs.
+    const int asked = split_len(k, splits, 64);
+    if ((k + asked - 1) / asked > 1 && workspace == nullptr) return hipErrorInvalidValue;
+    const StagedPlan p = staged_plan(m, n, k, splits);
+    const long long blocks = p.tiles * p.depth;
+    if (blocks > 0x7fffffffLL) return hipErrorInvalidValue;
+    const dim3 grid(static_cast<unsigned>(blocks));
+    float* ws = p.depth > 1 ? workspace : nullptr;
+    const auto run = [&](auto cfg) {
+        using Cfg = decltype(cfg);
+        hipLaunchKernelGGL((matmul_mfma16_staged<kBf16, kF32In, Cfg>), grid, dim3(Cfg::kThreads), 0, stream, a, b, c,
+                           m, n, k, p.k_split, ws);
+    };
+    // The form of a tile, by operand type (us on an MI355X, K = 2048 or 2040).
+    // 128x128: with at most one per CU two steps are loaded ahead (2048^2 fp32
+    // 42.7 against 48.5 with one; bf16 34.7 against 36.8), with more than one a
+    // second block per CU does better than the deeper prefetch (3072^2 fp32
+    // 100.4 against 114.3; bf16 80.8 against 85.6). Eight waves where the
+    // registers allow (bf16: 2048^2 34.7 against 44.3 with four; fp32 4096^2
+    // 141.8 on four waves against 154.9).
+    // 64x64 of 16-bit operands: two groups of waves, each taking every other K
+    // step, where there is one tile per CU at most (1024^2 14.6 against 18.0)
+    // and the caller's split count leaves the order of adds open; fp32
+    // operands are bound by the loads themselves and gain nothing.
+    const long long cus = std::max(device_cus(), 1);
+    if (p.bm == 128) {
+        if constexpr (kF32In) {
+            if (p.tiles <= cus) {
+                run(Staged<128, 128, 2, 2, 1, 2, 1>{});
+            } else {
+                run(Staged<128, 128, 2, 2, 1, 1, 2>{});
+            }
+        } else {
+            if (p.tiles <= cus) {
+                run(Staged<128, 128, 2, 4, 1, 2, 1>{});
+            } else {
+                run(Staged<128, 128, 2, 4, 1, 1, 1>{});
+            }
+        }
+    } else if (p.bm == 64) {
+        if (splits <= 1) {
+            run(Staged<64, 64, 2, 2, 1, 2, 2>{});
+        } else if (kF32In || p.tiles > cus) {
+            run(Staged<64, 64, 2, 2, 1, 2, 2, 4>{});
+        } else if constexpr (!kF32In) {
+            run(Staged<64, 64, 2, 2, 2, 2, 1, 4>{});
+        }
+    } else if (splits <= 1) {
+        run(Staged<32, 64, 1, 4, 1, 2, 2>{});
     } else {
-        hipLaunchKernelGGL((matmul_mfma16<kBf16, kF32In, false>), grid, dim3(256), 0, stream, a, b, c, m, n, k, k_split, ws);
+        run(Staged<32, 64, 1, 4, 1, 2, 2, 4>{});
     }
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess || depth == 1) return e;
-    return mchip_sum_split_partials(workspace, c, static_cast<std::size_t>(m) * n, depth, stream);
+    if (e != hipSuccess || p.depth == 1) return e;
+    return mchip_sum_split_partials(workspace, c, static_cast<std::size_t>(m) * n, p.depth, stream);
 }
 
 __global__ void __launch_bounds__(256) convert_kernel(const float* __restrict__ in, unsigned short* __restrict__ out,
@@ -473,7 +742,9 @@ extern "C" int mchip_launch_matmul_lowp(int kernel, int dtype, const void* a, co
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (m < 1 || n < 1 || k < 1) return hipErrorInvalidValue;
     if (kernel == kTensorCoreTf32) return hipErrorNotSupported;
-    const bool fast = fast_eligible(a, b, c, m, n, k, splits);
+    const int asked = split_len(k, splits, 64);
+    if ((k + asked - 1) / asked > 1 && workspace == nullptr) return hipErrorInvalidValue;
+    const bool fast = splits <= 1 && fast_eligible(a, b, c, m, n, k) && fast_preferred(m, n);
     if (kernel == kTensorCoreBf16 && dtype == MCHIP_DTYPE_BF16) {
         return fast ? launch_fast<true>(a, b, c, m, n, k, s) : launch16<true, false>(a, b, c, m, n, k, s, splits, workspace);
     }
@@ -529,7 +800,7 @@ extern "C" int mchip_launch_matmul_lowp_packed(int kernel, int dtype, const void
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (m < 1 || n < 1 || k < 1) return hipErrorInvalidValue;
     if (kernel == kTensorCoreTf32) return hipErrorNotSupported;
-    if (!fast_eligible(a_packed, b, c, m, n, k, 1)) return hipErrorInvalidValue;
+    if (!fast_eligible(a_packed, b, c, m, n, k)) return hipErrorInvalidValue;
     if (kernel == kTensorCoreBf16 && dtype == MCHIP_DTYPE_BF16) return launch_fast<true, true>(a_packed, b, c, m, n, k, s);
     if (kernel == kTensorCoreF16 && dtype == MCHIP_DTYPE_F16) return launch_fast<false, true>(a_packed, b, c, m, n, k, s);
     return hipErrorInvalidValue;
@@ -641,10 +912,9 @@ extern "C" int mchip_launch_mfma16_packed(int dtype, int shape, const void* a_pa
     return hipErrorInvalidValue;
 }
 
-extern "C" int mchip_tensor_core_k_ranges(int k, int splits) {
-    if (k < 1) return 0;
-    const int k_split = split_len(k, splits, kBK);
-    return std::max(1, (k + k_split - 1) / k_split);
+extern "C" int mchip_tensor_core_k_ranges(int m, int n, int k, int splits) {
+    if (m < 1 || n < 1 || k < 1) return 0;
+    return staged_plan(m, n, k, splits).depth;
 }
 
 extern "C" int mchip_mfma16_fast_fits(int m, int n, int k) {
@@ -666,10 +936,12 @@ extern "C" int mchip_matmul_blocks_per_cu(int kernel) {
     hipError_t e = hipErrorInvalidValue;
     switch (kernel) {
         case kTensorCoreBf16:
-            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, matmul_mfma16<true, true, true>, 256, 0);
+            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, matmul_mfma16_staged<true, true, Staged<128, 128, 2, 2, 1, 1, 2>>,
+                                                             256, 0);
             break;
         case kTensorCoreF16:
-            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, matmul_mfma16<false, true, true>, 256, 0);
+            e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, matmul_mfma16_staged<false, true, Staged<128, 128, 2, 2, 1, 1, 2>>,
+                                                             256, 0);
             break;
         default: return 2;
     }
