@@ -364,11 +364,12 @@ GemmEpilogueKernel generate_gemm_epilogue_kernel(const FusedProgram& program, st
           "int k_split, int depth, float* __restrict__ partial, unsigned* __restrict__ counters, McEpilogue epi)\n{\n"
        << unused << (constant ? "\t(void)k_split;\n" : "") << "\t(void)depth;\n"
        << (folds ? "" : "\t(void)counters;\n");
+    const char* ragged = fixed.ragged ? ", true" : "";
     if (body == GemmBody::F32Mfma) {
         os << "\tmc_gemm_f32_mfma<true, " << (vectorized_operands ? "true" : "false") << ">(a, b, c, " << mnk
            << ", " << (constant ? std::to_string(fixed.k_split) : std::string("k_split")) << ", partial, epi);\n}\n\n";
     } else if (is_narrow_body(body)) {
-        os << "\tmc_gemm_f32_narrow<" << narrow_config(body) << ">(a, b, c, "
+        os << "\tmc_gemm_f32_narrow<" << narrow_config(body) << ragged << ">(a, b, c, "
            << mnk << ", " << split << ", partial, counters, epi);\n}\n\n";
     } else {
         const char* cfg = body == GemmBody::F32RingBig    ? "McRingBig"
@@ -376,7 +377,7 @@ GemmEpilogueKernel generate_gemm_epilogue_kernel(const FusedProgram& program, st
                           : body == GemmBody::F32RingMid  ? "McRingMid"
                           : body == GemmBody::F32RingWide8 ? "McRingWide8"
                                                           : "McRingWide";
-        os << "\tmc_gemm_f32_ring<" << cfg << ">(a, b, c, "
+        os << "\tmc_gemm_f32_ring<" << cfg << ragged << ">(a, b, c, "
            << mnk << ", " << split << ", partial, counters, epi);\n}\n\n";
     }
     // Split K: the partial sums added in split order (a left fold from split

@@ -150,6 +150,7 @@ inline const char* narrow_config(GemmBody body) {
 // element) and ignores its m, n, k, k_split and depth arguments.
 struct GemmDims {
     int m = 0, n = 0, k = 0, k_split = 0, depth = 1;
+    bool ragged = false;  // the ragged form of a ring or narrow body
     int frag = 0;  // Bf16Frag, F16Frag: the tile shape (MCHIP_FRAG_*)
 };
 

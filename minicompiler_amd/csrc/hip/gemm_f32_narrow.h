@@ -39,6 +39,15 @@
 // per tile, in tile order). Rows past m read row m - 1 and
 // columns past n the last column chunk (every load in bounds); what they
 // produce is not stored.
+//
+// The ragged form (kRagged) takes any K of 16 or more (k_split still a
+// multiple of 16), any N of 4 or more and any float-aligned operands, without
+// counters. Its vector accesses go to 4-byte aligned addresses, which the
+// memory path takes; a chunk of columns that straddles n reads on into the
+// next row, except in the last rows of K: the last wave of the block that
+// holds the end of K loads its last K % 16 rows (16 when N alone is ragged)
+// float by float (past the last row of K or column of N the last one, so no
+// load is guarded), with zeros past K, before its other groups.
 #pragma once
 
 typedef float mc_nw_f32x4 __attribute__((ext_vector_type(4)));
@@ -55,10 +64,12 @@ struct McNarrowVec;
 template <>
 struct McNarrowVec<4> {
     typedef mc_nw_f32x4 type;
+    typedef float any __attribute__((ext_vector_type(4), aligned(4)));  // at any float address
 };
 template <>
 struct McNarrowVec<2> {
     typedef mc_nw_f32x2 type;
+    typedef float any __attribute__((ext_vector_type(2), aligned(4)));
 };
 
 // A configuration: kRG row groups of 16, kVec columns per lane and load
@@ -118,7 +129,7 @@ struct McNarrowRegs {
 // this block; the epilogue maps each value v of flat element i to what is
 // stored (out = C), or the raw sums go to `out` (a partial), added in the
 // launch when `counters` is given (not null).
-template <class Cfg, typename Epilogue>
+template <class Cfg, bool kRagged = false, typename Epilogue>
 __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, const float* __restrict__ b,
                                                    float* __restrict__ c, int m, int n, int k, int k_split,
                                                    int depth, float* __restrict__ partial, unsigned* __restrict__ counters,
@@ -142,13 +153,16 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
     const int bx = q % tiles_n, bz = (q / tiles_n) % tiles_m, by = q / (tiles_n * tiles_m);
     const int col0 = bx * Cfg::kCols;
     const int row0 = bz * Cfg::kRows;
-    const int colc = col0 + kVec * cl < n ? col0 + kVec * cl : n - kVec;
+    const int colc = col0 + kVec * cl < n ? col0 + kVec * cl : n - kVec;  // ragged: may straddle n
 
     // This wave's K range: the block's range cut into kW pieces of whole
     // 16-k groups (the last pieces may be empty).
     const int kb = by * k_split;
     const int ke = kb + k_split < k ? kb + k_split : k;
-    const int groups = (ke - kb) / 16;
+    // Ragged: the rows of K loaded float by float (the last wave's).
+    const int part = kRagged ? (ke - kb) % 16 : 0;
+    const int tail = kRagged && ke == k && (part != 0 || n % 4 != 0) ? (part != 0 ? part : 16) : 0;
+    const int groups = (ke - kb - tail) / 16;
     const int per = (groups + kW - 1) / kW;
     const int g0 = wave * per < groups ? wave * per : groups;
     const int g1 = g0 + per < groups ? g0 + per : groups;
@@ -220,6 +234,31 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
     // 32x64 tiles unsplit 18.5 / 20.2 us. The batching does not change the
     // order of the adds.
     McNarrowRegs<Cfg> x0, x1;
+    if constexpr (kRagged) {
+        if (tail != 0 && wave == kW - 1) {
+            const int k0 = k - tail;
+#pragma unroll
+            for (int r = 0; r < kRG; ++r) {
+                const int row = row0 + 16 * r + cl < m ? row0 + 16 * r + cl : m - 1;
+                const float* src = a + static_cast<long long>(row) * k + k0;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float v = src[4 * s + e < tail ? 4 * s + e : tail - 1];
+                    x0.a[0][r][e] = 4 * s + e < tail ? v : 0.0f;
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float* src = b + static_cast<long long>(k0 + (4 * s + e < tail ? 4 * s + e : tail - 1)) * n;
+#pragma unroll
+                for (int j = 0; j < kVec; ++j) {
+                    const float v = src[colc + j < n ? colc + j : n - 1];
+                    x0.b[0][e][j] = 4 * s + e < tail ? v : 0.0f;
+                }
+            }
+            compute(x0, McNarrowUnits<1>{});
+        }
+    }
     auto pipeline = [&](auto units) {
         constexpr int kN = decltype(units)::value;
         const int batches = (g1 - g0) / kN;
@@ -269,7 +308,7 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
     // then a chunk is stored float by float, the same values. Partials that
     // this launch adds go out as device-scope stores (mc_split_store).
     const bool fold = raw && counters != nullptr;
-    const bool vec_out = (reinterpret_cast<unsigned long long>(out) & (sizeof(BV) - 1)) == 0;
+    const bool vec_out = !kRagged && (reinterpret_cast<unsigned long long>(out) & (sizeof(BV) - 1)) == 0;
     // A lane's chunks (kRows 16 / kThreads of them, 1 to 4): all summed and
     // through the epilogue before the first store, so the epilogue's operand
     // loads of every chunk are in flight together, and a per-column operand
@@ -290,7 +329,8 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
         if (!raw && row < m && col < n) {
             const long long at = static_cast<long long>(row) * n + col;
 #pragma unroll
-            for (int j = 0; j < kVec; ++j) sum[j] = epilogue(sum[j], static_cast<unsigned>(at + j));
+            for (int j = 0; j < kVec; ++j)
+                if (!kRagged || col + j < n) sum[j] = epilogue(sum[j], static_cast<unsigned>(at + j));
         }
         sums[i] = sum;
     }
@@ -306,9 +346,12 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
             for (int j = 0; j < kVec; ++j) mc_split_store(out + at + j, sums[i][j]);
         } else if (vec_out) {
             *reinterpret_cast<BV*>(out + at) = sums[i];
+        } else if (kRagged && col + kVec <= n) {
+            *reinterpret_cast<typename McNarrowVec<kVec>::any*>(out + at) = sums[i];
         } else {
 #pragma unroll
-            for (int j = 0; j < kVec; ++j) out[at + j] = sums[i][j];
+            for (int j = 0; j < kVec; ++j)
+                if (!kRagged || col + j < n) out[at + j] = sums[i][j];
         }
     }
     if (!fold) return;

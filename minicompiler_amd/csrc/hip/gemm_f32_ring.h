@@ -18,6 +18,17 @@
 // Rows past M and columns past N are clamped to the last row / column
 // chunk, so every load is in bounds; what they bring only reaches C elements
 // that are not stored.
+//
+// The ragged form (kRagged, staged configurations) takes any K of 64 or more,
+// any N of 4 or more and any float-aligned operands, one unit per block, no
+// counters. Its 16-byte loads and 8-byte stores go to 4-byte aligned addresses,
+// which the memory path takes. A chunk of columns that straddles N reads on
+// into the next row (those C elements are not stored). Only the end of K needs
+// care: the unit that holds it loads its last K % 32 rows (32 when N alone is
+// ragged) float by float with zeros past K, in the prologue, as its first
+// step, so its latency is the first load's that every unit waits for anyway.
+// The order of the other steps is unchanged. On an MI355X, 2000x1001x1023 + bias
+// + ReLU: RAGGED_MEASUREMENTS
 #pragma once
 
 typedef float mc_ring_f32x4 __attribute__((ext_vector_type(4)));
@@ -144,8 +155,10 @@ struct McRingFetch {
     int b_step;
 };
 
+// `tail` (ragged): rows of K that the first step loads float by float; the
+// others start tail - 32 rows before them (step 0's place is never read there).
 struct McRingUnit {
-    int row0, col0, kb, steps, split;
+    int row0, col0, kb, steps, split, tail;
 };
 
 // A stage parity as a type, for the staged main loop's steps.
@@ -212,6 +225,41 @@ __device__ __forceinline__ void mc_ring_store_one(MC_RING_LDS unsigned char* wr,
     const int blk = idx < Cfg::kFA ? (wave * Cfg::kFA + idx) * 1024
                                    : Cfg::kABytes + (wave * Cfg::kFB + idx - Cfg::kFA) * 1024;
     *reinterpret_cast<MC_RING_LDS mc_ring_f32x4*>(wr + blk + 16 * lane) = v;
+}
+
+// A ragged unit's first step, its `tail` last rows of K (from k0), float by
+// float into the LDS positions a whole step's chunks take; zeros past them.
+template <class Cfg>
+__device__ __forceinline__ void mc_ring_fetch_tail(MC_RING_LDS unsigned char* wr, const float* __restrict__ a,
+                                                   const float* __restrict__ b, int m, int n, int k,
+                                                   const McRingUnit& u, int k0, int wave, int lane) {
+    mc_ring_f32x4 v[Cfg::kFetch];
+    // Past the last row of K or column of N, the last one is read (no load is
+    // guarded); rows past K become zeros.
+#pragma unroll
+    for (int idx = 0; idx < Cfg::kFetch; ++idx) {
+        if (idx < Cfg::kFA) {
+            const int rb = Cfg::kFA * wave + idx;
+            const int row = mc_ring_min(u.row0 + rb * 8 + (lane & 7), m - 1);
+            const int kk = 4 * (2 * (lane >> 4) + (((lane >> 3) & 1) ^ (rb & 1)));
+            const float* src = a + static_cast<long long>(row) * k + k0;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[idx][e] = src[mc_ring_min(kk + e, u.tail - 1)];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[idx][e] = kk + e < u.tail ? v[idx][e] : 0.0f;
+        } else {
+            constexpr int kLanesPerBRow = Cfg::kBRow / 16;
+            const int kk = (Cfg::kFB * wave + idx - Cfg::kFA) * (1024 / Cfg::kBRow) + lane / kLanesPerBRow;
+            const int col = u.col0 + 4 * ((lane % kLanesPerBRow) ^ (8 * ((kk >> 4) & 1)));
+            const float* src = b + static_cast<long long>(k0 + mc_ring_min(kk, u.tail - 1)) * n;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[idx][e] = src[mc_ring_min(col + e, n - 1)];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[idx][e] = kk < u.tail ? v[idx][e] : 0.0f;
+        }
+    }
+#pragma unroll
+    for (int idx = 0; idx < Cfg::kFetch; ++idx) mc_ring_store_one<Cfg>(wr, wave, lane, idx, v[idx]);
 }
 
 // All of a step's fetch instructions (the prologue's): direct loads, or for
@@ -370,7 +418,8 @@ __device__ __forceinline__ void mc_ring_barrier() {
 // sweep rows within 0.2%.
 // kSplit: raw partial sums that this launch adds, stored float by float
 // with device-scope stores (mc_split_store).
-template <class Cfg, bool kCheck, typename Epilogue, bool kSplit = false>
+// kEdge (ragged): a tile that reaches past N, stored float by float.
+template <class Cfg, bool kCheck, typename Epilogue, bool kSplit = false, bool kEdge = false>
 __device__ __forceinline__ void mc_ring_store(const mc_ring_f32x16 (&acc)[Cfg::kAI][Cfg::kBJ], float* __restrict__ out,
                                               int tile_row0, int tile_col0, int row0, int col, int m, int n, bool raw,
                                               const Epilogue& epilogue) {
@@ -385,6 +434,29 @@ __device__ __forceinline__ void mc_ring_store(const mc_ring_f32x16 (&acc)[Cfg::k
     const __amdgpu_buffer_rsrc_t c_rsrc = mc_ring_rsrc(out + static_cast<long long>(tile_row0) * n + tile_col0);
     const int c_off = 4 * ((row0 - tile_row0) * n + (col - tile_col0));
     auto row_step = [&](int i, int v) { return 4 * n * (32 * i + 8 * (v >> 2) + (v & 3)); };
+    if constexpr (kEdge) {
+#pragma unroll
+        for (int j = 0; j < Cfg::kBJ; ++j) {
+            if (col + j >= n) continue;
+#pragma unroll
+            for (int i = 0; i < Cfg::kAI; ++i) {
+                float o[16];
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const int row = row_of(i, v);
+                    if (row >= m) continue;
+                    const unsigned at =
+                        static_cast<unsigned>(row) * static_cast<unsigned>(n) + static_cast<unsigned>(col + j);
+                    o[v] = raw ? acc[i][j][v] : epilogue(acc[i][j][v], at);
+                }
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    if (row_of(i, v) < m) mc_ring_buffer_store(o[v], c_rsrc, c_off + 4 * j, row_step(i, v));
+                }
+            }
+        }
+        return;
+    }
     if constexpr (kSplit) {
 #pragma unroll
         for (int i = 0; i < Cfg::kAI; ++i)
@@ -492,12 +564,12 @@ __device__ __forceinline__ void mc_ring_fold(const float* __restrict__ partial, 
 // to `partial` (split s at s m n) and the epilogue is applied where the
 // splits are summed: in this launch, by the last block to finish a split of
 // the tile, when `counters` is given (not null), else by a separate launch.
-template <class Cfg, typename Epilogue>
+template <class Cfg, bool kRagged = false, typename Epilogue>
 __device__ __forceinline__ void mc_gemm_f32_ring(const float* __restrict__ a, const float* __restrict__ b,
                                                  float* __restrict__ c, int m, int n, int k, int k_split, int splits,
                                                  float* __restrict__ partial, unsigned* __restrict__ counters,
                                                  const Epilogue& epilogue) {
-    typedef McRingVec<Cfg::kBJ> BV;
+    static_assert(!kRagged || (Cfg::kStaged && Cfg::kStages == 2), "the ragged form's first step goes through registers");
     __shared__ __attribute__((aligned(1024))) unsigned char smem[Cfg::kLds];
     MC_RING_LDS unsigned char* lds = (MC_RING_LDS unsigned char*)(smem);  // generic -> LDS address space
 
@@ -532,6 +604,15 @@ __device__ __forceinline__ void mc_gemm_f32_ring(const float* __restrict__ a, co
         r.kb = r.split * k_split;
         const int ke = mc_ring_min(k, r.kb + k_split);
         r.steps = (ke - r.kb) / Cfg::kBK;
+        r.tail = 0;
+        if constexpr (kRagged) {
+            const int part = (ke - r.kb) % Cfg::kBK;
+            if (ke == k && (part != 0 || n % 4 != 0)) {
+                r.tail = part != 0 ? part : Cfg::kBK;
+                if (part != 0) ++r.steps;
+                r.kb -= Cfg::kBK;  // step t >= 1 is at kb + 32 t
+            }
+        }
         return r;
     };
     // A: wave w fills blocks rb = kFA w + i; lane l -> row 8 rb + l % 8,
@@ -557,7 +638,8 @@ __device__ __forceinline__ void mc_gemm_f32_ring(const float* __restrict__ a, co
         for (int i = 0; i < Cfg::kFB; ++i) {
             const int kk = (Cfg::kFB * wave + i) * (1024 / Cfg::kBRow) + lane / kLanesPerBRow;
             const int g = (lane % kLanesPerBRow) ^ (8 * ((kk >> 4) & 1));
-            const int col = mc_ring_min(u.col0 + 4 * g, n - 4);
+            int col = u.col0 + 4 * g;
+            if (kRagged ? col >= n : col > n - 4) col = n - 4;
             f.b_off[i] = 4 * (kk * n + col - u.col0);
         }
         f.b_step = 4 * Cfg::kBK * n;
@@ -592,6 +674,10 @@ __device__ __forceinline__ void mc_gemm_f32_ring(const float* __restrict__ a, co
     auto advance = [&]() {
         if (++ft == fu.steps) {
             ft = 0;
+            // Step 0 of a unit with a tail has no place in memory, unless it
+            // is the only one: then the unit's K range is not the first, and
+            // the 32 rows before it stand in for loads that nothing uses.
+            if constexpr (kRagged) ft = fu.tail != 0 && fu.steps > 1 ? 1 : 0;
             if (++fi < count) {
                 fu = unit_of(fi);
                 fetch = fetch_of(fu);
@@ -605,7 +691,11 @@ __device__ __forceinline__ void mc_gemm_f32_ring(const float* __restrict__ a, co
     int issued = 0;
     const int pre = mc_ring_min(total, Cfg::kStages - 1);
     for (; issued < pre; ++issued) {
-        mc_ring_fetch<Cfg>(lds + ws * Cfg::kStage, fetch, wave, ft);
+        if (kRagged && fu.tail != 0) {
+            mc_ring_fetch_tail<Cfg>(lds + ws * Cfg::kStage, a, b, m, n, k, fu, k - fu.tail, wave, lane);
+        } else {
+            mc_ring_fetch<Cfg>(lds + ws * Cfg::kStage, fetch, wave, ft);
+        }
         ws = next(ws);
         advance();
     }
@@ -700,7 +790,10 @@ __device__ __forceinline__ void mc_gemm_f32_ring(const float* __restrict__ a, co
         if (col < n) {
             float* __restrict__ out = splits > 1 ? partial + static_cast<long long>(u.split) * m * n : c;
             const int r0 = u.row0 + wr + 4 * half;
-            if (fold) {
+            if (kRagged && u.col0 + Cfg::kBN > n) {
+                mc_ring_store<Cfg, true, Epilogue, false, true>(acc, out, u.row0, u.col0, r0, col, m, n, splits > 1,
+                                                                epilogue);
+            } else if (fold) {
                 if (u.row0 + Cfg::kBM <= m)
                     mc_ring_store<Cfg, false, Epilogue, true>(acc, out, u.row0, u.col0, r0, col, m, n, true, epilogue);
                 else

@@ -92,6 +92,7 @@ struct Launch {
     unsigned grid_x = 0, grid_y = 0, grid_z = 0, sum_grid = 0, block = 256;
     int k_split = 0, depth = 1;
     GemmBody body = GemmBody::F32Mfma;
+    bool ragged = false;  // the ragged form of a ring or narrow body
     const void* a_ptr = nullptr;
     const void* b_ptr = nullptr;
     void* c_ptr = nullptr;
@@ -642,8 +643,14 @@ private:
         if (l.matmul == MatmulKernel::SplitK &&
             (l.ring_cfg == MCHIP_RING_NONE || l.ring_cfg == MCHIP_RING_NARROW)) {
             int shape = 0, splits = 0, k_split = 0;
-            if (mchip_f32_narrow_plan(l.m, l.n, l.k, std::max(l.splits, 1), device_.cu_count,
-                                      l.ring_cfg == MCHIP_RING_NARROW, &shape, &splits, &k_split)) {
+            const bool force = l.ring_cfg == MCHIP_RING_NARROW;
+            bool narrow = mchip_f32_narrow_plan(l.m, l.n, l.k, std::max(l.splits, 1), device_.cu_count, force, &shape,
+                                                &splits, &k_split) != 0;
+            if (!narrow && !force && (l.n % 4 != 0 || l.k % 16 != 0)) {
+                narrow = l.ragged = mchip_f32_ragged_narrow_plan(l.m, l.n, l.k, std::max(l.splits, 1), device_.cu_count,
+                                                                 &shape, &splits, &k_split) != 0;
+            }
+            if (narrow) {
                 l.k_split = k_split;
                 l.depth = splits;
                 switch (shape) {
@@ -656,7 +663,7 @@ private:
             }
         }
         split_layout(l.k, l.splits, &l.k_split, &l.depth);
-        if (l.matmul == MatmulKernel::Vectorized || l.k % 4 != 0) return GemmBody::F32Mfma;
+        if (l.matmul == MatmulKernel::Vectorized) return GemmBody::F32Mfma;
         unsigned grid = 0, block = 0;
         switch (mchip_f32_ring_plan_cfg(l.m, l.n, l.k, l.depth, device_.cu_count, l.ring_cfg, &grid, &block)) {
             case MCHIP_RING_BIG: return GemmBody::F32RingBig;
@@ -670,8 +677,14 @@ private:
                 l.ring_cfg = MCHIP_RING_WIDE;
                 return GemmBody::F32RingWide;
             case MCHIP_RING_MID: return GemmBody::F32RingMid;
-            default: return GemmBody::F32Mfma;
+            default: break;
         }
+        if (l.ring_cfg == MCHIP_RING_NONE &&
+            mchip_f32_ragged_ring_plan(l.m, l.n, l.k, l.depth, device_.cu_count, &grid, &block) != MCHIP_RING_NONE) {
+            l.ragged = true;  // 4-wave blocks, with a group in the store (as above)
+            return GemmBody::F32RingWide;
+        }
+        return GemmBody::F32Mfma;
     }
 
     // The fused elementwise group this matmul's store can apply, or kNoNode.
@@ -749,6 +762,7 @@ private:
                 dims.n = l.n;
                 dims.k = l.lowp ? l.kp : l.k;
                 dims.frag = l.frag;
+                dims.ragged = l.ragged;
                 dims.k_split = l.k_split;
                 dims.depth = l.depth;
                 k.source = generate_gemm_epilogue_kernel(*f.fused, acc, shapes, f.type.shape, l.n % 4 == 0 && l.k % 4 == 0,
@@ -819,7 +833,12 @@ private:
                     l.block = 256;
                 } else {
                     unsigned grid = 0, block = 0;
-                    mchip_f32_ring_plan_cfg(l.m, l.n, l.k, l.depth, device_.cu_count, l.ring_cfg, &grid, &block);
+                    if (l.ragged) {
+                        mchip_f32_ragged_ring_plan(l.m, l.n, l.k, l.depth, device_.cu_count, &grid, &block);
+                        block = 256;
+                    } else {
+                        mchip_f32_ring_plan_cfg(l.m, l.n, l.k, l.depth, device_.cu_count, l.ring_cfg, &grid, &block);
+                    }
                     l.grid_x = grid;
                     l.grid_y = l.grid_z = 1;
                     l.block = block;
@@ -828,7 +847,7 @@ private:
                 l.sum_grid = static_cast<unsigned>(std::max<std::size_t>(
                     1, std::min<std::size_t>((static_cast<std::size_t>(l.count) + 255) / 256, 8192)));
                 l.partial = l.depth > 1 ? l.workspace : nullptr;
-                l.fold = l.depth > 1 && l.counters != nullptr && l.body != GemmBody::F32Mfma;
+                l.fold = l.depth > 1 && l.counters != nullptr && l.body != GemmBody::F32Mfma && !l.ragged;
                 if (!l.fold) l.counters = nullptr;
                 l.epilogue_inputs.assign(graph_.node(l.epilogue_node).inputs.size(), nullptr);
                 continue;

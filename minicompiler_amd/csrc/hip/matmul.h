@@ -150,6 +150,17 @@ int mchip_narrow_cols(int shape);
 int mchip_f32_narrow_plan(int m, int n, int k, int max_splits, int cu_count, int force, int* shape, int* splits,
                           int* k_split);
 
+/* The ragged forms of the ring (128x128 tiles) and narrow bodies, for what
+ * the exact ones do not take: N not a multiple of 4, K not of 32 (16), or
+ * operands not 16-byte aligned (any float address). The ring's from K 64 and
+ * N 4 on (MCHIP_RING_WIDE, MCHIP_RING_WIDE8 or MCHIP_RING_NONE; one block
+ * per tile and split), the narrow body's as mchip_f32_narrow_plan decides
+ * for N and K rounded up, from K 16 and N 4 on. Smaller ones stay on the
+ * two-stage body. They do not add splits in the launch. */
+int mchip_f32_ragged_ring_plan(int m, int n, int k, int depth, int cu_count, unsigned* grid, unsigned* block);
+int mchip_f32_ragged_narrow_plan(int m, int n, int k, int max_splits, int cu_count, int* shape, int* splits,
+                                 int* k_split);
+
 /* The narrow-tile body directly: `rows` 16 (m <= 16) or 32, K in `splits`
  * ranges; above one range the partials go to `workspace` (splits * m * n
  * floats) and are summed in range order. */

@@ -164,11 +164,11 @@ using RingThin = McRingThin;
 using RingMid = McRingMid;
 constexpr int kRBKRing = RingWide::kBK;
 
-template <class Cfg, int kBlocksPerCu>
+template <class Cfg, int kBlocksPerCu, bool kRagged = false>
 __global__ void __launch_bounds__(Cfg::kThreads, kBlocksPerCu)
     matmul_ring_f32(const float* __restrict__ a, const float* __restrict__ b, float* __restrict__ c, int m, int n,
                     int k, int k_split, int depth, float* __restrict__ partial, unsigned* __restrict__ counters) {
-    mc_gemm_f32_ring<Cfg>(a, b, c, m, n, k, k_split, depth, partial, counters, McGemmStore{});
+    mc_gemm_f32_ring<Cfg, kRagged>(a, b, c, m, n, k, k_split, depth, partial, counters, McGemmStore{});
 }
 
 // ---------------------------------------------------------------- narrow tiles
@@ -177,13 +177,13 @@ struct McIdentity {
     __device__ __forceinline__ float operator()(float v, unsigned) const { return v; }
 };
 
-template <class Cfg>
+template <class Cfg, bool kRagged>
 __global__ void __launch_bounds__(Cfg::kThreads) matmul_narrow_f32(const float* __restrict__ a,
                                                                     const float* __restrict__ b, float* __restrict__ c,
                                                                     int m, int n, int k, int k_split, int depth,
                                                                     float* __restrict__ partial,
                                                                     unsigned* __restrict__ counters) {
-    mc_gemm_f32_narrow<Cfg>(a, b, c, m, n, k, k_split, depth, partial, counters, McIdentity{});
+    mc_gemm_f32_narrow<Cfg, kRagged>(a, b, c, m, n, k, k_split, depth, partial, counters, McIdentity{});
 }
 
 // ---------------------------------------------------------------- split-K sum
@@ -246,10 +246,15 @@ int device_cu_count() {
 
 template <class Cfg>
 void narrow_kernel(const float* a, const float* b, float* c, int m, int n, int k, hipStream_t s, int k_split,
-                   int depth, float* part, unsigned* counters) {
+                   int depth, float* part, unsigned* counters, bool ragged) {
     const dim3 grid(((n + Cfg::kCols - 1) / Cfg::kCols) * depth * ((m + Cfg::kRows - 1) / Cfg::kRows));
-    hipLaunchKernelGGL((matmul_narrow_f32<Cfg>), grid, dim3(Cfg::kThreads), 0, s, a, b, c, m, n, k, k_split, depth,
-                       part, counters);
+    if (ragged) {
+        hipLaunchKernelGGL((matmul_narrow_f32<Cfg, true>), grid, dim3(Cfg::kThreads), 0, s, a, b, c, m, n, k, k_split,
+                           depth, part, counters);
+    } else {
+        hipLaunchKernelGGL((matmul_narrow_f32<Cfg, false>), grid, dim3(Cfg::kThreads), 0, s, a, b, c, m, n, k, k_split,
+                           depth, part, counters);
+    }
 }
 
 // The narrow-tile body in tile shape `shape` on `depth` K ranges of
@@ -257,18 +262,20 @@ void narrow_kernel(const float* a, const float* b, float* c, int m, int n, int k
 // the launch when `counters` (zeroed, one per tile) is given, else by a
 // separate launch.
 int launch_narrow(const float* a, const float* b, float* c, int m, int n, int k, hipStream_t s, int shape,
-                  int k_split, int depth, float* workspace, unsigned* counters) {
+                  int k_split, int depth, float* workspace, unsigned* counters, bool ragged = false) {
     float* dst = depth > 1 ? workspace : c;
-    if (!aligned16(a) || !aligned16(b) || dst == nullptr) return hipErrorInvalidValue;
+    if ((!ragged && (!aligned16(a) || !aligned16(b))) || dst == nullptr) return hipErrorInvalidValue;
     if (shape == MCHIP_NARROW_16X64_STREAM && m > 16) return hipErrorInvalidValue;
     float* part = depth > 1 ? workspace : nullptr;
-    unsigned* ctr = depth > 1 ? counters : nullptr;
+    unsigned* ctr = depth > 1 && !ragged ? counters : nullptr;
     switch (shape) {
-        case MCHIP_NARROW_32X64: narrow_kernel<McNarrow32>(a, b, c, m, n, k, s, k_split, depth, part, ctr); break;
-        case MCHIP_NARROW_16X64_STREAM: narrow_kernel<McNarrow16>(a, b, c, m, n, k, s, k_split, depth, part, ctr); break;
-        case MCHIP_NARROW_16X64: narrow_kernel<McNarrow16x64>(a, b, c, m, n, k, s, k_split, depth, part, ctr); break;
-        case MCHIP_NARROW_16X32: narrow_kernel<McNarrow16x32>(a, b, c, m, n, k, s, k_split, depth, part, ctr); break;
-        case MCHIP_NARROW_64X64: narrow_kernel<McNarrow64>(a, b, c, m, n, k, s, k_split, depth, part, ctr); break;
+        case MCHIP_NARROW_32X64: narrow_kernel<McNarrow32>(a, b, c, m, n, k, s, k_split, depth, part, ctr, ragged); break;
+        case MCHIP_NARROW_16X64_STREAM:
+            narrow_kernel<McNarrow16>(a, b, c, m, n, k, s, k_split, depth, part, ctr, ragged);
+            break;
+        case MCHIP_NARROW_16X64: narrow_kernel<McNarrow16x64>(a, b, c, m, n, k, s, k_split, depth, part, ctr, ragged); break;
+        case MCHIP_NARROW_16X32: narrow_kernel<McNarrow16x32>(a, b, c, m, n, k, s, k_split, depth, part, ctr, ragged); break;
+        case MCHIP_NARROW_64X64: narrow_kernel<McNarrow64>(a, b, c, m, n, k, s, k_split, depth, part, ctr, ragged); break;
         default: return hipErrorInvalidValue;
     }
     const hipError_t e = hipGetLastError();
@@ -287,9 +294,12 @@ struct MfmaPlan {
     int k_split = 0, depth = 1;
     unsigned ring_grid = 0, ring_block = 0;
     bool vec = false;
+    bool ragged = false;  // the ragged form of the narrow or ring body
     // The split's partials go to a workspace and a body that can add them
     // in its own launch (ring or narrow) runs it.
-    bool can_fold() const { return status == hipSuccess && depth > 1 && (narrow || ring != MCHIP_RING_NONE); }
+    bool can_fold() const {
+        return status == hipSuccess && depth > 1 && !ragged && (narrow || ring != MCHIP_RING_NONE);
+    }
 };
 
 MfmaPlan plan_mfma_f32(bool double_buffer, bool a16, bool b16, bool c16, bool ws16, bool has_ws, int m, int n, int k,
@@ -297,11 +307,15 @@ MfmaPlan plan_mfma_f32(bool double_buffer, bool a16, bool b16, bool c16, bool ws
     MfmaPlan p;
     // split_k on the narrow-tile body when the plan (or the caller) takes it,
     // with at most the caller's split count (its workspace's size).
-    if (split_k && (ring_cfg == MCHIP_RING_NONE || ring_cfg == MCHIP_RING_NARROW) && a16 && b16) {
+    if (split_k && (ring_cfg == MCHIP_RING_NONE || ring_cfg == MCHIP_RING_NARROW)) {
         int shape = 0, ns = 0, nk = 0;
-        if (mchip_f32_narrow_plan(m, n, k, std::max(splits, 1), device_cu_count(), ring_cfg == MCHIP_RING_NARROW,
-                                  &shape, &ns, &nk)) {
-            p.narrow = true;
+        const int cus = device_cu_count();
+        const bool force = ring_cfg == MCHIP_RING_NARROW;
+        p.narrow = a16 && b16 && mchip_f32_narrow_plan(m, n, k, std::max(splits, 1), cus, force, &shape, &ns, &nk);
+        if (!p.narrow && !force && (!a16 || !b16 || n % 4 != 0 || k % 16 != 0)) {
+            p.narrow = p.ragged = mchip_f32_ragged_narrow_plan(m, n, k, std::max(splits, 1), cus, &shape, &ns, &nk);
+        }
+        if (p.narrow) {
             p.shape = shape;
             p.k_split = nk;
             p.depth = ns;
@@ -328,6 +342,10 @@ MfmaPlan plan_mfma_f32(bool double_buffer, bool a16, bool b16, bool c16, bool ws
                  ? mchip_f32_ring_plan_cfg(m, n, k, p.depth, device_cu_count(), ring_cfg, &p.ring_grid, &p.ring_block)
                  : MCHIP_RING_NONE;
     if (ring_cfg != MCHIP_RING_NONE && p.ring != ring_cfg) p.status = hipErrorInvalidValue;
+    if (double_buffer && ring_cfg == MCHIP_RING_NONE && p.ring == MCHIP_RING_NONE) {
+        p.ring = mchip_f32_ragged_ring_plan(m, n, k, p.depth, device_cu_count(), &p.ring_grid, &p.ring_block);
+        p.ragged = p.ring != MCHIP_RING_NONE;
+    }
     return p;
 }
 
@@ -339,7 +357,7 @@ int launch_mfma_f32(bool double_buffer, const float* a, const float* b, float* c
     const MfmaPlan p = plan_mfma_f32(double_buffer, aligned16(a), aligned16(b), aligned16(c), aligned16(workspace),
                                      workspace != nullptr, m, n, k, splits, ring_cfg, split_k);
     if (p.status != hipSuccess) return p.status;
-    if (p.narrow) return launch_narrow(a, b, c, m, n, k, stream, p.shape, p.k_split, p.depth, workspace, counters);
+    if (p.narrow) return launch_narrow(a, b, c, m, n, k, stream, p.shape, p.k_split, p.depth, workspace, counters, p.ragged);
     const int k_split = p.k_split, depth = p.depth;
     const dim3 grid((n + kMBN - 1) / kMBN, (m + kMBM - 1) / kMBM, depth);
     const bool vec = p.vec;
@@ -348,7 +366,13 @@ int launch_mfma_f32(bool double_buffer, const float* a, const float* b, float* c
     const int ring = p.ring;
     // The ring's fold stores C 16 bytes at a time.
     unsigned* ctr = p.can_fold() && aligned16(c) ? counters : nullptr;
-    if (ring == MCHIP_RING_THIN) {
+    if (p.ragged && ring == MCHIP_RING_WIDE8) {
+        hipLaunchKernelGGL((matmul_ring_f32<RingWide8, 1, true>), dim3(ring_grid), dim3(ring_block), 0, stream, a, b, c,
+                           m, n, k, k_split, depth, out_ws, ctr);
+    } else if (p.ragged) {
+        hipLaunchKernelGGL((matmul_ring_f32<RingWide, 2, true>), dim3(ring_grid), dim3(ring_block), 0, stream, a, b, c,
+                           m, n, k, k_split, depth, out_ws, ctr);
+    } else if (ring == MCHIP_RING_THIN) {
         hipLaunchKernelGGL((matmul_ring_f32<RingThin, 1>), dim3(ring_grid), dim3(ring_block), 0, stream, a, b, c, m, n,
                            k, k_split, depth, out_ws, ctr);
     } else if (ring == MCHIP_RING_BIG) {
@@ -453,6 +477,36 @@ extern "C" int mchip_f32_ring_plan_cfg(int m, int n, int k, int depth, int cu_co
 
 extern "C" int mchip_f32_ring_plan(int m, int n, int k, int depth, int cu_count, unsigned* grid, unsigned* block) {
     return mchip_f32_ring_plan_cfg(m, n, k, depth, cu_count, MCHIP_RING_NONE, grid, block);
+}
+
+extern "C" int mchip_f32_ragged_ring_plan(int m, int n, int k, int depth, int cu_count, unsigned* grid,
+                                          unsigned* block) {
+    *grid = 0;
+    *block = 0;
+    // Loads of whole chunks need 4 columns and, in every K range but a
+    // one-step last one, a step of 32 before the last rows of K.
+    if (m < 1 || n < 4 || k < 64 || depth < 1 || cu_count < 1) return MCHIP_RING_NONE;
+    unsigned g = 0, b = 0;
+    const long long k32 = (static_cast<long long>(k) + 31) / 32 * 32, n4 = (static_cast<long long>(n) + 3) / 4 * 4;
+    if (k32 >= (1LL << 31) || n4 >= (1LL << 31)) return MCHIP_RING_NONE;
+    if (mchip_f32_ring_plan_cfg(m, static_cast<int>(n4), static_cast<int>(k32), depth, cu_count, MCHIP_RING_WIDE, &g,
+                                &b) == MCHIP_RING_NONE) {
+        return MCHIP_RING_NONE;  // byte offsets past 31 bits
+    }
+    // One block per tile-split: 4-wave blocks, two to a CU, or the 8-wave
+    // block where there is at most one per CU (as the exact plan).
+    const long long units = (static_cast<long long>(m) + 127) / 128 * ((static_cast<long long>(n) + 127) / 128) * depth;
+    if (units > 0x7fffffffLL) return MCHIP_RING_NONE;
+    *grid = static_cast<unsigned>(units);
+    *block = units <= cu_count ? RingWide8::kThreads : RingWide::kThreads;
+    return units <= cu_count ? MCHIP_RING_WIDE8 : MCHIP_RING_WIDE;
+}
+
+extern "C" int mchip_f32_ragged_narrow_plan(int m, int n, int k, int max_splits, int cu_count, int* shape, int* splits,
+                                            int* k_split) {
+    *shape = *splits = *k_split = 0;
+    if (m < 1 || n < 4 || k < 16 || n > 0x7ffffff0 || k > 0x7ffffff0) return 0;
+    return mchip_f32_narrow_plan(m, (n + 3) / 4 * 4, (k + 15) / 16 * 16, max_splits, cu_count, 0, shape, splits, k_split);
 }
 
 extern "C" int mchip_narrow_rows(int shape) {

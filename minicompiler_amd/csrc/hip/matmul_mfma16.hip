@@ -238,16 +238,27 @@ __global__ void __launch_bounds__(Cfg::kThreads, Cfg::kBlocks) matmul_mfma16_sta
             r.b[e] = *reinterpret_cast<const BV*>(b_src + static_cast<std::ptrdiff_t>(k0 + e) * n);
         __builtin_amdgcn_sched_barrier(0);
     };
+    // Element by element, zeros past ke. The loads are clamped to the last k
+    // and column instead of guarded (32 branches, each a live mask).
     auto load_part = [&](Regs& r, int k0) {
 #pragma unroll
         for (int i = 0; i < kALoads; ++i)
 #pragma unroll
-            for (int e = 0; e < kAK; ++e) r.a[i][e] = k0 + kAK * ac + e < ke ? a_src[i][k0 + e] : T(0);
+            for (int e = 0; e < kAK; ++e) {
+                const int kk = k0 + kAK * ac + e;
+                const T v = a_src[i][min(kk, ke - 1) - kAK * ac];
+                r.a[i][e] = kk < ke ? v : T(0);
+            }
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
+        for (int e = 0; e < 8; ++e) {
+            const int kk = k0 + 8 * bk + e;
+            const T* const src = b + static_cast<std::ptrdiff_t>(min(kk, ke - 1)) * n;
 #pragma unroll
-            for (int j = 0; j < kCV; ++j)
-                r.b[e][j] = k0 + 8 * bk + e < ke && bcol + j < n ? b_src[static_cast<std::ptrdiff_t>(k0 + e) * n + j] : T(0);
+            for (int j = 0; j < kCV; ++j) {
+                const T v = src[min(bcol + j, n - 1)];
+                r.b[e][j] = kk < ke ? v : T(0);
+            }
+        }
     };
     auto store = [&](const Regs& r, int stage) {
         unsigned char* const s = stages + stage * Cfg::kStagePitch;

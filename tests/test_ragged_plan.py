@@ -1,0 +1,34 @@
+"""Which body runs an FP32 product that the exact ring and narrow forms do not
+take (host logic, no GPU)."""
+
+import ctypes
+
+import pytest
+
+NONE, WIDE, WIDE8 = 0, 1, 6
+
+
+@pytest.mark.parametrize("m,n,k,depth,want", [
+    (2000, 1001, 1023, 1, (WIDE8, 128, 512)),   # 16 x 8 tiles: one per CU at most
+    (3648, 2176, 423, 1, (WIDE, 493, 256)),
+    (1000, 1000, 1000, 4, (WIDE8, 256, 512)),
+    (128, 4, 64, 1, (WIDE8, 1, 512)),
+    (128, 3, 64, 1, (NONE, 0, 0)), (128, 4, 63, 1, (NONE, 0, 0)),  # the two-stage body's
+    (64, 2 << 20, 33, 1, (NONE, 0, 0)),
+])
+def test_the_ragged_ring_runs_one_block_per_tile_and_split(mc, m, n, k, depth, want):
+    f = mc.library().mchip_f32_ragged_ring_plan
+    grid, block = ctypes.c_uint(), ctypes.c_uint()
+    assert (f(m, n, k, depth, 256, ctypes.byref(grid), ctypes.byref(block)), grid.value, block.value) == want
+
+
+@pytest.mark.parametrize("m,n,k,splits,want", [
+    (16, 1001, 777, 8, (1, 7, 112)),   # as 16x1004x784
+    (256, 513, 2047, 8, (2, 1, 2048)),
+    (8, 3, 100, 1, None), (8, 4, 15, 1, None),
+])
+def test_the_ragged_narrow_plan_is_the_exact_one_rounded_up(mc, m, n, k, splits, want):
+    f = mc.library().mchip_f32_ragged_narrow_plan
+    out = [ctypes.c_int() for _ in range(3)]
+    ok = f(m, n, k, splits, 256, *[ctypes.byref(x) for x in out])
+    assert (tuple(x.value for x in out) if ok else None) == want
