@@ -716,7 +716,7 @@ MC_API int mc_kernel_sources(const void* h, char* out, int size) {
             const FusedProgram p = n.op == OpKind::FusedElementwise ? *n.fused : hip::single_op_program(n.op);
             std::vector<Shape> shapes;
             for (NodeId in : n.inputs) shapes.push_back(c->graph.node(in).type.shape);
-            sources.push_back(hip::generate_elementwise_kernel(p, shapes, n.type.shape, cg).source);
+            sources.push_back(hip::generate_graph_kernel(p, shapes, n.type.shape, cg).source);
         }
     }
     std::string all;

@@ -562,4 +562,261 @@ ElementwiseKernel generate_elementwise_kernel(const FusedProgram& program, const
     return k;
 }
 
+namespace {
+
+// How the column form reads one input for a vector of four output elements
+// starting at element 4 p.
+struct ColumnAccess {
+    enum class Kind {
+        Vector,    // contiguous: vector p
+        Scalar,    // one element
+        Hoisted,   // a periodic row whose period divides the item spacing: read once per lane
+        Rows,      // periodic or general, constant over runs of `run` >= 4 elements: one or two loads
+        Inner,     // general, contiguous along a last dimension that is a multiple of 4: a vector
+        Elements,  // anything else: four loads
+    } kind = Kind::Vector;
+    std::size_t period = 0, run = 0;
+};
+
+std::size_t gcd(std::size_t a, std::size_t b) { return b == 0 ? a : gcd(b, a % b); }
+std::size_t lcm(std::size_t a, std::size_t b) { return a / gcd(a, b) * b; }
+
+// The column form, for broadcast inputs and counts that are not a multiple
+// of 4. Bound: HBM. What kept the flat form from it: reading a broadcast row
+// again for every item (with its modulo), and scalar accesses, four times
+// the memory instructions, wherever a vector could straddle a period or a
+// row or the count was odd. Here
+// - accesses are 16-byte vectors whatever the count (its last one to three
+//   elements are done by one lane each of the first block);
+// - a lane's items are spaced Q vectors apart, Q x 4 a multiple of the rows'
+//   periods, so its columns are the same in every item: a periodic row is
+//   read once per lane (element by element when the period is not a multiple
+//   of 4) and kept in registers. Lanes are numbered flat, lane t of group
+//   t / Q taking vectors U Q (t / Q) + t % Q + u Q, so no lane is idle and a
+//   wave's vectors are consecutive except where a group ends; Q is a multiple
+//   of 8 (128 bytes) where the tensor has the rows for it;
+// - an input that is constant along the last dimensions ([M, 1] beside
+//   [M, N]) is one load per vector, two and a select where a vector may
+//   straddle two rows.
+// Measured on an MI355X, against the flat form: BatchNorm + ReLU [50177, 129]
+// 17.9 -> 11.3 us, [31168, 483] 37.3 -> 23, [200704, 256] 6.19 -> 6.34 TB/s; a
+// row-wise normalisation with [M, 1] statistics, [8192, 2048], 32.3 -> 22.2 us
+// (a copy of its size: 21.5). Items per lane: 4 best or within 2% of it on all
+// of these among 2, 4, 8 and 16.
+ElementwiseKernel generate_column_kernel(const FusedProgram& program, const std::vector<Shape>& input_shapes,
+                                         const Shape& out_shape, const CodegenOptions& options) {
+    const std::size_t num_inputs = input_shapes.size();
+    const std::size_t numel = num_elements(out_shape), nv = numel / 4, rem = numel % 4;
+    std::vector<Access> access;
+    for (const Shape& s : input_shapes) access.push_back(classify_access(s, out_shape));
+
+    // Items per lane: as the flat form, but no more than leave four waves of
+    // lanes to each of 256 CUs.
+    const std::size_t most = program.num_ops() >= 8 ? 8 : 4;
+    const std::size_t items =
+        options.items_per_lane > 0 ? options.items_per_lane : std::max<std::size_t>(1, std::min(most, nv / 65536));
+
+    // Item spacing in vectors: the periods that still leave a lane its items.
+    std::size_t q = 1;
+    std::vector<ColumnAccess> cols(num_inputs);
+    for (std::size_t k = 0; k < num_inputs; ++k) {
+        const Access& a = access[k];
+        ColumnAccess& c = cols[k];
+        switch (a.kind) {
+            case Access::Kind::Contiguous: c.kind = ColumnAccess::Kind::Vector; break;
+            case Access::Kind::Scalar: c.kind = ColumnAccess::Kind::Scalar; break;
+            case Access::Kind::Periodic: {
+                c.period = a.period;
+                const std::size_t with = lcm(q, a.period / gcd(a.period, 4));
+                c.kind = ColumnAccess::Kind::Elements;
+                if (items > 1 && with * items <= nv) {
+                    q = with;
+                    c.kind = ColumnAccess::Kind::Hoisted;
+                } else if (a.period % 4 == 0) {
+                    c.kind = ColumnAccess::Kind::Inner;
+                }
+                break;
+            }
+            case Access::Kind::General: {
+                const std::vector<std::int64_t> strides = broadcast_strides(input_shapes[k], out_shape);
+                c.run = 1;
+                for (std::size_t d = out_shape.size(); d-- > 0 && strides[d] == 0;) c.run *= static_cast<std::size_t>(out_shape[d]);
+                const bool whole = !out_shape.empty() && out_shape.back() % 4 == 0;
+                c.kind = c.run >= 4                          ? ColumnAccess::Kind::Rows
+                         : whole && strides.back() == 1 ? ColumnAccess::Kind::Inner
+                                                        : ColumnAccess::Kind::Elements;
+                break;
+            }
+        }
+    }
+    // Whole 128-byte lines per segment where the tensor is long enough, and
+    // at least a block's lanes.
+    if (lcm(q, 8) * items <= nv) q = lcm(q, 8);
+    if (q < kElementwiseBlock) q *= (kElementwiseBlock + q - 1) / q;
+    const std::size_t groups = (nv + q * items - 1) / (q * items);
+    const std::size_t lanes = groups * q;
+
+    std::ostringstream os;
+    os << "// minicompiler-hip elementwise kernel: " << program.num_ops() << " op(s), out f32"
+       << to_string(out_shape) << ", 16-byte vector accesses, " << items << " item(s) per lane " << q
+       << " vectors apart.\n";
+    os << "typedef float mc_f32x4 __attribute__((ext_vector_type(4)));\n\n";
+    os << program_function(program, num_inputs);
+    // The element a general or periodic input supplies for output element i.
+    for (std::size_t k = 0; k < num_inputs; ++k) {
+        if (access[k].kind != Access::Kind::General && access[k].kind != Access::Kind::Periodic) continue;
+        os << "__device__ __forceinline__ unsigned mc_index_" << k << "(unsigned i) { return "
+           << (access[k].kind == Access::Kind::General ? access[k].index : "i % " + u32(access[k].period)) << "; }\n";
+    }
+    os << "extern \"C\" __global__ void __launch_bounds__(" << kElementwiseBlock << ")\n"
+       << kElementwiseKernelName << "(float* __restrict__ out";
+    for (std::size_t k = 0; k < num_inputs; ++k) os << ", const float* __restrict__ in" << k;
+    os << ", unsigned n)\n{\n";
+    for (std::size_t k = 0; k < num_inputs; ++k) {
+        if (cols[k].kind == ColumnAccess::Kind::Scalar) os << "\tconst float s" << k << " = in" << k << "[0];\n";
+    }
+    const std::string Q = u32(q), U = u32(items);
+    const std::string ld = options.nontemporal_loads ? "__builtin_nontemporal_load(" : "*(";
+    auto vec = [&](std::size_t k) { return "reinterpret_cast<const mc_f32x4*>(in" + std::to_string(k) + ")"; };
+    auto element = [&](std::size_t k, const std::string& i) {
+        return "in" + std::to_string(k) + "[mc_index_" + std::to_string(k) + "(" + i + ")]";
+    };
+    auto four = [&](std::size_t k, const std::string& i) {
+        if (access[k].kind == Access::Kind::Periodic && access[k].period > 4) {
+            return "mc_wrap4<" + u32(access[k].period) + ">(in" + std::to_string(k) + ", " + i + ")";
+        }
+        return "mc_f32x4{" + element(k, i) + ", " + element(k, i + " + 1u") + ", " + element(k, i + " + 2u") + ", " +
+               element(k, i + " + 3u") + "}";
+    };
+    // Input k's vector p, in registers before the arithmetic.
+    auto load = [&](std::size_t k) -> std::string {
+        const ColumnAccess& c = cols[k];
+        switch (c.kind) {
+            case ColumnAccess::Kind::Vector: return ld + vec(k) + " + p)";
+            case ColumnAccess::Kind::Inner:
+                return "*reinterpret_cast<const mc_f32x4*>(in" + std::to_string(k) + " + mc_index_" + std::to_string(k) +
+                       "(4u * p))";
+            case ColumnAccess::Kind::Rows: {
+                if (c.run % 4 == 0) return "mc_f32x4(" + element(k, "4u * p") + ")";
+                const std::string two = "mc_straddle<" + u32(c.run) + ">(4u * p, " + element(k, "4u * p") + ", " +
+                                        element(k, "4u * p + 3u") + ")";
+                return two;
+            }
+            default: return four(k, "4u * p");
+        }
+    };
+    auto value = [&](std::size_t k, const char* lane) -> std::string {
+        switch (cols[k].kind) {
+            case ColumnAccess::Kind::Scalar: return "s" + std::to_string(k);
+            case ColumnAccess::Kind::Hoisted: return "h" + std::to_string(k) + lane;
+            default: return "a" + std::to_string(k) + "[u]" + lane;
+        }
+    };
+    auto in_registers = [&](std::size_t k) {
+        return cols[k].kind == ColumnAccess::Kind::Scalar || cols[k].kind == ColumnAccess::Kind::Hoisted;
+    };
+    auto emit_items = [&](const std::string& indent, bool checked) {
+        const std::string head = "#pragma unroll\n" + indent + "for (unsigned u = 0; u < " + U + "; ++u) {\n" + indent +
+                                 "\tconst unsigned p = base + u * " + Q + ";\n" +
+                                 (checked ? indent + "\tif (p >= " + u32(nv) + ") break;\n" : std::string());
+        for (std::size_t k = 0; k < num_inputs; ++k) {
+            if (!in_registers(k)) os << indent << "mc_f32x4 a" << k << "[" << items << "];\n";
+        }
+        os << indent << head;
+        for (std::size_t k = 0; k < num_inputs; ++k) {
+            if (!in_registers(k)) os << indent << "\ta" << k << "[u] = " << load(k) << ";\n";
+        }
+        os << indent << "}\n" << indent << head << indent << "\tmc_f32x4 o;\n";
+        for (const char* lane : {".x", ".y", ".z", ".w"}) {
+            os << indent << "\to" << lane << " = mc_program(";
+            for (std::size_t k = 0; k < num_inputs; ++k) os << (k ? ", " : "") << value(k, lane);
+            os << ");\n";
+        }
+        const std::string at = "reinterpret_cast<mc_f32x4*>(out) + p";
+        os << indent << "\t"
+           << (options.nontemporal_stores ? "__builtin_nontemporal_store(o, " + at + ");" : "*(" + at + ") = o;") << "\n";
+        // Each item's store before the next item's arithmetic, as in the flat form.
+        os << indent << "\t__builtin_amdgcn_sched_barrier(0);\n" << indent << "}\n";
+    };
+    os << "\tfor (unsigned t = blockIdx.x * " << u32(kElementwiseBlock) << " + threadIdx.x; t < " << u32(lanes)
+       << "; t += gridDim.x * " << u32(kElementwiseBlock) << ") {\n"
+       << "\t\tconst unsigned base = t + t / " << Q << " * " << u32((items - 1) * q) << ";\n";
+    for (std::size_t k = 0; k < num_inputs; ++k) {
+        if (cols[k].kind != ColumnAccess::Kind::Hoisted) continue;
+        os << "\t\tconst mc_f32x4 h" << k << " = ";
+        if (cols[k].period % 4 == 0) {
+            os << vec(k) << "[base % " << u32(cols[k].period / 4) << "];\n";
+        } else {
+            os << four(k, "4u * base") << ";\n";
+        }
+    }
+    os << "\t\tif (base + " << u32((items - 1) * q) << " < " << u32(nv) << ") {\n";
+    emit_items("\t\t\t", false);
+    os << "\t\t} else {\n";
+    emit_items("\t\t\t", true);
+    os << "\t\t}\n\t}\n";
+    if (rem != 0) {
+        os << "\tif (blockIdx.x == 0 && threadIdx.x < " << u32(rem) << ") {\n\t\tconst unsigned i = " << u32(4 * nv)
+           << " + threadIdx.x;\n\t\tout[i] = mc_program(";
+        for (std::size_t k = 0; k < num_inputs; ++k) {
+            if (k) os << ", ";
+            const Access::Kind kind = access[k].kind;
+            os << (kind == Access::Kind::Scalar       ? "s" + std::to_string(k)
+                   : kind == Access::Kind::Contiguous ? "in" + std::to_string(k) + "[i]"
+                                                      : element(k, "i"));
+        }
+        os << ");\n\t}\n";
+    }
+    os << "\t(void)n;\n}\n";
+    std::string text = os.str();
+    if (text.find("mc_wrap4") != std::string::npos) {
+        // Elements i .. i + 3 of a row that repeats every kPeriod > 4 elements: one
+        // 16-byte load at any float address, moved back from the row's end where
+        // it would cross it, and the row's first elements in the places past it
+        // (four loads of 4 bytes, 16 bytes apart across the lanes, took as long
+        // in the memory pipe as all of a lane's streaming: BatchNorm [50177, 129]
+        // 12.9 us so, 11.3 with this).
+        text.insert(text.find("__device__ __forceinline__ unsigned mc_index_"),
+                    "typedef float mc_f32x4u __attribute__((ext_vector_type(4), aligned(4)));\n"
+                    "template <unsigned kPeriod>\n__device__ __forceinline__ mc_f32x4 mc_wrap4(const float* "
+                    "__restrict__ in, unsigned i)\n{\n\tconst unsigned at = i % kPeriod;\n\tconst unsigned from = at < "
+                    "kPeriod - 4u ? at : kPeriod - 4u;\n\tconst unsigned past = at - from;\n\tconst mc_f32x4 v = "
+                    "*reinterpret_cast<const mc_f32x4u*>(in + from);\n\tconst float a = in[0], b = in[1], c = in[2];\n"
+                    "\treturn mc_f32x4{past == 0u ? v.x : past == 1u ? v.y : past == 2u ? v.z : v.w,\n"
+                    "\t\tpast == 0u ? v.y : past == 1u ? v.z : past == 2u ? v.w : a,\n"
+                    "\t\tpast == 0u ? v.z : past == 1u ? v.w : past == 2u ? a : b,\n"
+                    "\t\tpast == 0u ? v.w : past == 1u ? a : past == 2u ? b : c};\n}\n");
+    }
+    if (text.find("mc_straddle") != std::string::npos) {
+        // Element i + e of a vector at i, for an input constant over runs of
+        // kRun elements: the first run's value or, past its end, the next's.
+        text.insert(text.find("__device__ __forceinline__ unsigned mc_index_"),
+                    "template <unsigned kRun>\n__device__ __forceinline__ mc_f32x4 mc_straddle(unsigned i, float first, "
+                    "float next)\n{\n\tconst unsigned left = kRun - i % kRun;\n\treturn mc_f32x4{first, 1u < left ? "
+                    "first : next, 2u < left ? first : next, 3u < left ? first : next};\n}\n");
+    }
+    ElementwiseKernel k;
+    k.source = std::move(text);
+    k.vectorized = true;
+    k.items_per_lane = static_cast<unsigned>(items);
+    k.lanes = lanes;
+    return k;
+}
+
+}  // namespace
+
+ElementwiseKernel generate_graph_kernel(const FusedProgram& program, const std::vector<Shape>& input_shapes,
+                                        const Shape& out_shape, const CodegenOptions& options) {
+    const std::size_t numel = num_elements(out_shape);
+    bool column = numel % 4 != 0;
+    for (const Shape& s : input_shapes) {
+        const Access::Kind kind = classify_access(s, out_shape).kind;
+        column = column || kind == Access::Kind::Periodic || kind == Access::Kind::General;
+    }
+    if (options.allow_vectorize && column && numel >= 1024) {
+        return generate_column_kernel(program, input_shapes, out_shape, options);
+    }
+    return generate_elementwise_kernel(program, input_shapes, out_shape, options);
+}
+
 }  // namespace minicompiler::hip

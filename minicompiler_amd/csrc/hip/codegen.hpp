@@ -47,6 +47,9 @@ struct ElementwiseKernel {
     std::string source;
     bool vectorized = false;
     unsigned items_per_lane = 1;
+    // The grid's lanes for the column form (one step each), whose `n` argument
+    // counts floats; 0 for the flat form.
+    std::size_t lanes = 0;
     // Elements (or vectors) one block covers per step of its loop.
     unsigned items_per_block_step() const { return kElementwiseBlock * items_per_lane; }
 };
@@ -68,6 +71,13 @@ Access classify_access(const Shape& in, const Shape& out);
 
 ElementwiseKernel generate_elementwise_kernel(const FusedProgram& program, const std::vector<Shape>& input_shapes,
                                               const Shape& out_shape, const CodegenOptions& options = {});
+
+// The kernel a compiled graph runs for an elementwise node: the column form
+// (codegen.cpp, generate_column_kernel) for 1024 elements or more with a
+// broadcast input or a count that is not a multiple of 4, else
+// generate_elementwise_kernel's.
+ElementwiseKernel generate_graph_kernel(const FusedProgram& program, const std::vector<Shape>& input_shapes,
+                                        const Shape& out_shape, const CodegenOptions& options = {});
 
 inline constexpr const char* kGemmEpilogueKernelName = "mc_gemm_epilogue";
 inline constexpr const char* kSumSplitsEpilogueKernelName = "mc_sum_splits_epilogue";

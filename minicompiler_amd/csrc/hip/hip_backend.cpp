@@ -777,7 +777,7 @@ private:
                 node.op == OpKind::FusedElementwise ? *node.fused : single_op_program(node.op);
             std::vector<Shape> shapes;
             for (NodeId in : node.inputs) shapes.push_back(graph_.node(in).type.shape);
-            jobs.push_back({j, generate_elementwise_kernel(program, shapes, node.type.shape, cg)});
+            jobs.push_back({j, generate_graph_kernel(program, shapes, node.type.shape, cg)});
         }
         const std::string arch = arch_base(device_.arch);
         const int dev = options_.device;
@@ -854,7 +854,7 @@ private:
             }
             const std::size_t numel = graph_.node(l.node).type.num_elements();
             l.function = built[j]->function;
-            l.count = static_cast<unsigned>(kern.vectorized ? numel / 4 : numel);
+            l.count = static_cast<unsigned>(kern.vectorized && kern.lanes == 0 ? numel / 4 : numel);
             // Blocks per CU of the grid (those past what fits at once run in
             // turn), capped by the work: by default enough for one loop step
             // per block up to 64 per CU. A block that stores and exits lets a
@@ -865,7 +865,8 @@ private:
             int per_cu = static_cast<int>(options_.elementwise_blocks_per_cu);
             if (per_cu == 0) per_cu = kElementwiseBlocksPerCu;
             const std::size_t per_step = kern.items_per_block_step();
-            const std::size_t needed = (static_cast<std::size_t>(l.count) + per_step - 1) / per_step;
+            const std::size_t needed = kern.lanes > 0 ? (kern.lanes + kElementwiseBlock - 1) / kElementwiseBlock
+                                                      : (static_cast<std::size_t>(l.count) + per_step - 1) / per_step;
             const std::size_t resident = std::max<std::size_t>(1, static_cast<std::size_t>(per_cu) * device_.cu_count);
             l.grid = static_cast<unsigned>(std::max<std::size_t>(1, std::min(needed, resident)));
             l.ptrs.assign(1 + graph_.node(l.node).inputs.size(), nullptr);

@@ -146,7 +146,7 @@ int main(int argc, char** argv) {
             for (NodeId in : n.inputs) shapes.push_back(opt->node(in).type.shape);
             hip::CodegenOptions cg;
             cg.allow_vectorize = hopt.vectorize;
-            std::cout << "// node " << n.name << "\n" << hip::generate_elementwise_kernel(p, shapes, n.type.shape, cg).source;
+            std::cout << "// node " << n.name << "\n" << hip::generate_graph_kernel(p, shapes, n.type.shape, cg).source;
         }
     }
     if (!run && !bench) return 0;
