@@ -357,6 +357,7 @@ GemmEpilogueKernel generate_gemm_epilogue_kernel(const FusedProgram& program, st
     }
     const char* bounds = body == GemmBody::F32RingBig || body == GemmBody::F32RingThin ? "256, 1"
                          : body == GemmBody::F32RingWide8                              ? "512, 1"
+                         : body == GemmBody::F32Narrow16x16                            ? "512"
                          : is_narrow_body(body)                                        ? "256"
                                                                                        : "256, 2";
     os << "extern \"C\" __global__ void __launch_bounds__(" << bounds << ")\n" << kGemmEpilogueKernelName

@@ -99,6 +99,7 @@ enum class GemmBody {
     F32Narrow16x64,  // likewise, 16x64 tiles for M > 16 (short K, more tiles than 32x64 give)
     F32Narrow16x32,  // likewise, 16x32 tiles
     F32Narrow64,  // likewise, 64x64 tiles
+    F32Narrow16x16,  // likewise, 16x16 tiles, 8 waves (short K, few tiles)
     Bf16Fast,     // bf16 operands in HBM, 256x256 tiles, 512 lanes, one block per tile
     F16Fast,      // fp16 operands, likewise
     Bf16Packed,   // bf16, the same tiles, both operands packed
@@ -114,7 +115,7 @@ inline bool is_bf16_body(GemmBody body) {
 
 inline bool is_narrow_body(GemmBody body) {
     return body == GemmBody::F32Narrow16 || body == GemmBody::F32Narrow32 || body == GemmBody::F32Narrow16x64 ||
-           body == GemmBody::F32Narrow16x32 || body == GemmBody::F32Narrow64;
+           body == GemmBody::F32Narrow16x32 || body == GemmBody::F32Narrow64 || body == GemmBody::F32Narrow16x16;
 }
 
 inline bool is_f32_body(GemmBody body) {
@@ -127,13 +128,17 @@ inline bool is_f32_body(GemmBody body) {
 inline int narrow_rows(GemmBody body) {
     return body == GemmBody::F32Narrow64 ? 64 : body == GemmBody::F32Narrow32 ? 32 : 16;
 }
-inline int narrow_cols(GemmBody body) { return body == GemmBody::F32Narrow16x32 ? 32 : 64; }
+inline int narrow_cols(GemmBody body) {
+    return body == GemmBody::F32Narrow16x16 ? 16 : body == GemmBody::F32Narrow16x32 ? 32 : 64;
+}
+inline unsigned narrow_threads(GemmBody body) { return body == GemmBody::F32Narrow16x16 ? 512 : 256; }
 inline const char* narrow_config(GemmBody body) {
     switch (body) {
         case GemmBody::F32Narrow16: return "McNarrow16";
         case GemmBody::F32Narrow16x64: return "McNarrow16x64";
         case GemmBody::F32Narrow16x32: return "McNarrow16x32";
         case GemmBody::F32Narrow64: return "McNarrow64";
+        case GemmBody::F32Narrow16x16: return "McNarrow16x16";
         default: return "McNarrow32";
     }
 }

@@ -1,5 +1,5 @@
 // FP32 GEMM body for narrow tiles: C tiles of 16 kRG rows x 16 kVec columns
-// (32x64, 16x64 or 16x32) on v_mfma_f32_16x16x4f32, for products too small
+// (64x64 down to 16x16) on v_mfma_f32_16x16x4f32, for products too small
 // or too thin to fill the chip
 // with the ring body's 128x128 and 256x256 tiles (M <= 16, where B is read
 // once and HBM is the bound; and products of a few million outputs or
@@ -20,7 +20,7 @@
 // blocks (mapped to logical blocks XCD by XCD, below); its kW
 // waves cut that range into consecutive pieces, one accumulator set each.
 // Lane l of a wave has k slot s = l / 16 and index c = l % 16. For each group
-// of 16 k from kg the lane loads (V = kVec, 4 or 2 columns per lane)
+// of 16 k from kg the lane loads (V = kVec, 4, 2 or 1 columns per lane)
 //   A[16 r + c][kg + 4s .. kg + 4s + 3]              for row group r < kRG
 //   B[kg + 4s + e][col0 + V c .. col0 + V c + V - 1] for e = 0..3
 // and MFMA (r, e, j) takes A load r's element e and B load e's element j:
@@ -62,6 +62,11 @@ struct McNarrowUnits {
 template <int kVec>
 struct McNarrowVec;
 template <>
+struct McNarrowVec<1> {
+    typedef float type __attribute__((ext_vector_type(1)));
+    typedef float any __attribute__((ext_vector_type(1)));
+};
+template <>
 struct McNarrowVec<4> {
     typedef mc_nw_f32x4 type;
     typedef float any __attribute__((ext_vector_type(4), aligned(4)));  // at any float address
@@ -78,9 +83,12 @@ struct McNarrowVec<2> {
 // are non-temporal (a read-only stream reached 7.1 TB/s with them against
 // 6.3 TB/s without on an MI355X). kRedRows: rows of the LDS array the waves
 // add their tiles through (at least kRows); more than kRows only to keep a
-// second block off the CU (LDS is 160 KiB per CU).
-template <int kRG_, int kVec_, int kW_, int kU_, bool kStreamB_, int kRedRows_ = 16 * kRG_>
+// second block off the CU (LDS is 160 KiB per CU); kAcc: accumulators per
+// element (a power of two), MFMA e of a group adding to accumulator e % kAcc
+// (8: the groups of every second batch to the other four), summed pairwise.
+template <int kRG_, int kVec_, int kW_, int kU_, bool kStreamB_, int kRedRows_ = 16 * kRG_, int kAcc_ = 1>
 struct McNarrowCfg {
+    static constexpr int kAcc = kAcc_;
     static constexpr int kRG = kRG_, kVec = kVec_, kW = kW_, kU = kU_;
     static constexpr bool kStreamB = kStreamB_;
     static constexpr int kRows = 16 * kRG, kCols = 16 * kVec, kThreads = 64 * kW;
@@ -88,12 +96,12 @@ struct McNarrowCfg {
     static_assert(kRedRows >= kRows, "the reduction holds a whole tile");
 };
 
-// The configurations the library runs, 4 waves each, batches of up to 2
-// groups: 16x64 tiles for M <= 16 (B streamed), 32x64 tiles, and for
+// The configurations the library runs, 4 waves each and batches of up to 2
+// groups but for the last one: 16x64 tiles for M <= 16 (B streamed), 32x64 tiles, and for
 // short-K products that these would leave with half the CUs idle, 16x64 and
-// 16x32 tiles. At one K range every configuration adds the same products in
-// the same order (per element: the 4 waves' pieces of K in wave order, each
-// a chain of 16x16x4 MFMAs), so they give the same bits.
+// 16x32 tiles. At one K range each of the 4-wave configurations adds the
+// same products in the same order (per element: the 4 waves' pieces of K in
+// wave order, each a chain of 16x16x4 MFMAs), so they give the same bits.
 using McNarrow16 = McNarrowCfg<1, 4, 4, 2, true>;
 using McNarrow32 = McNarrowCfg<2, 4, 4, 2, false>;
 using McNarrow16x64 = McNarrowCfg<1, 4, 4, 2, false>;
@@ -104,8 +112,18 @@ using McNarrow16x32 = McNarrowCfg<1, 2, 4, 2, false>;
 // With 512 tiles (two per CU, 1024x2048x512) two co-resident blocks took
 // 31-36 us against 22.5 us for one block per CU in two rounds.
 using McNarrow64 = McNarrowCfg<4, 4, 4, 2, false, 96>;
+// 16x16 tiles, eight waves: for products that any other shape would have to
+// split over K ranges, and K short enough that a block's 128 bytes per k (16
+// rows of A, 16 columns of B, at about 45 GB/s per CU) cost less than the
+// ranges' sum launch (mchip_f32_narrow_plan). Eight accumulators per element:
+// a wave's chain of adds is as short as with the ranges, and the error no
+// larger (relative in the 2-norm, ranges / four accumulators / eight:
+// 1x512x2048 1.37e-7 / 1.58e-7 / 1.22e-7, 16x4096x1024 1.55e-7 / 1.20e-7 /
+// 1.00e-7). Batches of one group: 2, 4 and 8 groups were no faster
+// (1x512x2048 5.9 us against 6.1, 6.2 and 6.7).
+using McNarrow16x16 = McNarrowCfg<1, 1, 8, 1, false, 16, 8>;
 
-// A 16- or 8-byte buffer load at (voffset + soffset) from the resource's
+// A 16-, 8- or 4-byte buffer load at (voffset + soffset) from the resource's
 // base; kStream: non-temporal (the slc bit: a read-only stream reached 7.1
 // TB/s with non-temporal loads against 6.3 TB/s without on an MI355X).
 template <typename T, bool kStream>
@@ -113,8 +131,10 @@ __device__ __forceinline__ T mc_narrow_load(__amdgpu_buffer_rsrc_t rsrc, int vof
     constexpr int kAux = kStream ? 2 : 0;
     if constexpr (sizeof(T) == 16)
         return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b128(rsrc, voffset, soffset, kAux));
-    else
+    else if constexpr (sizeof(T) == 8)
         return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(rsrc, voffset, soffset, kAux));
+    else
+        return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(rsrc, voffset, soffset, kAux));
 }
 
 // One batch of a wave's operands: kU groups of 16 k.
@@ -143,14 +163,23 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
     // The grid is one-dimensional: block L runs on XCD L % 8 (the hardware
     // hands consecutive workgroups to the 8 XCDs in turn). With the count a
     // multiple of 8, XCD x takes the x-th contiguous eighth of the blocks in
-    // (column tile, row tile, K range) order, so the blocks sharing an L2
-    // share K ranges of A and B (one range per XCD when there are 8).
+    // (column tile, row tile, K range) order, or with the row tiles first
+    // where B is the larger operand, so the blocks sharing an L2 share K
+    // ranges of A and B (one range per XCD when there are 8) and an L2 reads
+    // all of the smaller operand and a share of the larger (4 MB: on
+    // an MI355X 100x2048x512 7.0 us with the columns first, 5.7 so;
+    // 128x2048x1024 12.2 and 8.3).
     const int tiles_n = (n + Cfg::kCols - 1) / Cfg::kCols;
     const int tiles_m = (m + Cfg::kRows - 1) / Cfg::kRows;
     const int total = static_cast<int>(gridDim.x);
     const int L = static_cast<int>(blockIdx.x);
     const int q = total % 8 == 0 ? (L % 8) * (total / 8) + L / 8 : L;
-    const int bx = q % tiles_n, bz = (q / tiles_n) % tiles_m, by = q / (tiles_n * tiles_m);
+    const bool rows_first = m < n && tiles_m > 1;
+    const int inner = rows_first ? tiles_m : tiles_n;
+    const int outer = rows_first ? tiles_n : tiles_m;
+    const int rest = q / inner, by = rest / outer;
+    const int bx = rows_first ? rest - by * outer : q - rest * inner;
+    const int bz = rows_first ? q - rest * inner : rest - by * outer;
     const int col0 = bx * Cfg::kCols;
     const int row0 = bz * Cfg::kRows;
     const int colc = col0 + kVec * cl < n ? col0 + kVec * cl : n - kVec;  // ragged: may straddle n
@@ -186,7 +215,14 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
     const int b_off = 4 * (4 * s * n + colc - col0);
     const int b_row = 4 * n;  // bytes per row of B
 
-    mc_nw_f32x4 acc[kRG][kVec] = {};
+    // The ragged form keeps several accumulators too: the two-stage body it
+    // replaces split K into more ranges than these tiles need, and with as
+    // many partial sums the rounding error is no larger. Relative error in
+    // the 2-norm and time on an MI355X, the two-stage body / one accumulator
+    // / these: 449x1263x1472 2.9e-7 39.1 us / 3.5e-7 29.0 us / 2.5e-7 30.6 us,
+    // 64x2032x1327 1.9e-7 19.0 us / 3.3e-7 8.7 us / 1.7e-7 8.7 us.
+    constexpr int kAcc = Cfg::kAcc > 1 || !kRagged ? Cfg::kAcc : kRG * kVec <= 8 ? 4 : 2;
+    mc_nw_f32x4 part_acc[kAcc][kRG][kVec] = {};
     // Loads of `units` groups from group g into x, then (after a scheduling
     // barrier: left to itself the scheduler interleaves each load with the
     // MFMAs that use it and waits for it there) nothing else.
@@ -203,9 +239,11 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
         __builtin_amdgcn_sched_barrier(0);
     };
     // The MFMAs of `units` groups held in x: MFMA (u, e, r, j) multiplies A
-    // load (u, r)'s element e by B load (u, e)'s element j.
-    auto compute = [&](const McNarrowRegs<Cfg>& x, auto units) {
+    // load (u, r)'s element e by B load (u, e)'s element j. `set`: 0 or 1, the
+    // register set, for eight accumulators.
+    auto compute = [&](const McNarrowRegs<Cfg>& x, auto units, auto set) {
         constexpr int kN = decltype(units)::value;
+        constexpr int kFirst = 4 * decltype(set)::value;
 #pragma unroll
         for (int u = 0; u < kN; ++u)
 #pragma unroll
@@ -214,7 +252,8 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
                 for (int r = 0; r < kRG; ++r)
 #pragma unroll
                     for (int j = 0; j < kVec; ++j)
-                        acc[r][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.a[u][r][e], x.b[u][e][j], acc[r][j], 0, 0, 0);
+                        part_acc[(kFirst + e) % kAcc][r][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                            x.a[u][r][e], x.b[u][e][j], part_acc[(kFirst + e) % kAcc][r][j], 0, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
     };
     // Whole batches, software-pipelined over two register sets: the loads of
@@ -235,29 +274,30 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
     // order of the adds.
     McNarrowRegs<Cfg> x0, x1;
     if constexpr (kRagged) {
-        if (tail != 0 && wave == kW - 1) {
-            const int k0 = k - tail;
+        // Every wave runs it, all but the block's last one on zeros: under a
+        // condition the compiler kept two copies of the accumulators.
+        const int mine = wave == kW - 1 ? tail : 0;
+        const int rows = mine > 0 ? mine : 1;
+        auto at = [&](int i) { return k - rows + (i < rows ? i : rows - 1); };
 #pragma unroll
-            for (int r = 0; r < kRG; ++r) {
-                const int row = row0 + 16 * r + cl < m ? row0 + 16 * r + cl : m - 1;
-                const float* src = a + static_cast<long long>(row) * k + k0;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float v = src[4 * s + e < tail ? 4 * s + e : tail - 1];
-                    x0.a[0][r][e] = 4 * s + e < tail ? v : 0.0f;
-                }
-            }
+        for (int r = 0; r < kRG; ++r) {
+            const int row = row0 + 16 * r + cl < m ? row0 + 16 * r + cl : m - 1;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const float* src = b + static_cast<long long>(k0 + (4 * s + e < tail ? 4 * s + e : tail - 1)) * n;
-#pragma unroll
-                for (int j = 0; j < kVec; ++j) {
-                    const float v = src[colc + j < n ? colc + j : n - 1];
-                    x0.b[0][e][j] = 4 * s + e < tail ? v : 0.0f;
-                }
+                const float v = a[static_cast<long long>(row) * k + at(4 * s + e)];
+                x0.a[0][r][e] = 4 * s + e < mine ? v : 0.0f;
             }
-            compute(x0, McNarrowUnits<1>{});
         }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float* src = b + static_cast<long long>(at(4 * s + e)) * n;
+#pragma unroll
+            for (int j = 0; j < kVec; ++j) {
+                const float v = src[colc + j < n ? colc + j : n - 1];
+                x0.b[0][e][j] = 4 * s + e < mine ? v : 0.0f;
+            }
+        }
+        compute(x0, McNarrowUnits<1>{}, McNarrowUnits<0>{});
     }
     auto pipeline = [&](auto units) {
         constexpr int kN = decltype(units)::value;
@@ -267,21 +307,21 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
             load(x0, g0, units);
             for (; i + 2 < batches; i += 2) {
                 load(x1, g0 + (i + 1) * kN, units);
-                compute(x0, units);
+                compute(x0, units, McNarrowUnits<0>{});
                 load(x0, g0 + (i + 2) * kN, units);
-                compute(x1, units);
+                compute(x1, units, McNarrowUnits<1>{});
             }
             if (batches - i == 2) {
                 load(x1, g0 + (i + 1) * kN, units);
-                compute(x0, units);
-                compute(x1, units);
+                compute(x0, units, McNarrowUnits<0>{});
+                compute(x1, units, McNarrowUnits<1>{});
             } else {
-                compute(x0, units);
+                compute(x0, units, McNarrowUnits<0>{});
             }
         }
         for (int g = g0 + batches * kN; g < g1; ++g) {
             load(x0, g, McNarrowUnits<1>{});
-            compute(x0, McNarrowUnits<1>{});
+            compute(x0, McNarrowUnits<1>{}, McNarrowUnits<0>{});
         }
     };
     if (kU > 1 && per >= 32 && (depth > 1 || kRG == 1)) {
@@ -290,6 +330,15 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
         pipeline(McNarrowUnits<1>{});
     }
 
+    mc_nw_f32x4(&acc)[kRG][kVec] = part_acc[0];
+#pragma unroll
+    for (int step = 1; step < kAcc; step *= 2)
+#pragma unroll
+        for (int i = 0; i < kAcc; i += 2 * step)
+#pragma unroll
+            for (int r = 0; r < kRG; ++r)
+#pragma unroll
+                for (int j = 0; j < kVec; ++j) part_acc[i][r][j] += part_acc[i + step][r][j];
     // Lane l holds rows 16 r + 4s + v of column chunk cl.
 #pragma unroll
     for (int r = 0; r < kRG; ++r)
@@ -301,7 +350,7 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
             red[wave][16 * r + 4 * s + v][cl] = o;
         }
     __syncthreads();
-    // The tile's chunks, summed over the waves in wave order.
+    // The tile's chunks, summed over the waves (one accumulator: in wave order).
     const bool raw = depth > 1;
     float* __restrict__ out = raw ? partial + static_cast<long long>(by) * m * n : c;
     // C or a partial may sit at any 4-byte address (a caller's workspace):
@@ -315,16 +364,29 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
     // (a bias: every chunk of a lane is in the same columns) is loaded once;
     // chunk by chunk, the compiler loaded it again and waited for it in each
     // chunk, after the previous chunk's store.
-    constexpr int kChunks = Cfg::kRows * 16 / Cfg::kThreads;
-    static_assert(kChunks * Cfg::kThreads == Cfg::kRows * 16, "a whole number of chunks per lane");
+    constexpr int kAll = Cfg::kRows * 16;
+    constexpr int kChunks = (kAll + Cfg::kThreads - 1) / Cfg::kThreads;
+    static_assert(kAll % Cfg::kThreads == 0 || kChunks == 1, "a whole number of chunks per lane, or one for some lanes");
     BV sums[kChunks];
 #pragma unroll
     for (int i = 0; i < kChunks; ++i) {
         const int t = static_cast<int>(threadIdx.x) + i * Cfg::kThreads;
+        if (t >= kAll) continue;
         const int r = t >> 4, ch = t & 15;
         BV sum = red[0][r][ch];
+        if constexpr (kAcc > 1) {  // sums of its own: pairwise over the waves too
+            BV w[kW];
 #pragma unroll
-        for (int w = 1; w < kW; ++w) sum += red[w][r][ch];
+            for (int i2 = 0; i2 < kW; ++i2) w[i2] = red[i2][r][ch];
+#pragma unroll
+            for (int step = 1; step < kW; step *= 2)
+#pragma unroll
+                for (int i2 = 0; i2 + step < kW; i2 += 2 * step) w[i2] += w[i2 + step];
+            sum = w[0];
+        } else {
+#pragma unroll
+            for (int w = 1; w < kW; ++w) sum += red[w][r][ch];
+        }
         const int row = row0 + r, col = col0 + kVec * ch;
         if (!raw && row < m && col < n) {
             const long long at = static_cast<long long>(row) * n + col;
@@ -339,7 +401,7 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
         const int t = static_cast<int>(threadIdx.x) + i * Cfg::kThreads;
         const int r = t >> 4, ch = t & 15;
         const int row = row0 + r, col = col0 + kVec * ch;
-        if (row >= m || col >= n) continue;
+        if (t >= kAll || row >= m || col >= n) continue;
         const long long at = static_cast<long long>(row) * n + col;
         if (fold) {
 #pragma unroll

@@ -658,6 +658,7 @@ private:
                     case MCHIP_NARROW_16X64: return GemmBody::F32Narrow16x64;
                     case MCHIP_NARROW_16X32: return GemmBody::F32Narrow16x32;
                     case MCHIP_NARROW_64X64: return GemmBody::F32Narrow64;
+                    case MCHIP_NARROW_16X16: return GemmBody::F32Narrow16x16;
                     default: return GemmBody::F32Narrow32;
                 }
             }
@@ -830,7 +831,7 @@ private:
                     const int rows = narrow_rows(l.body), cols = narrow_cols(l.body);
                     l.grid_x = static_cast<unsigned>(((l.n + cols - 1) / cols) * l.depth * ((l.m + rows - 1) / rows));
                     l.grid_y = l.grid_z = 1;
-                    l.block = 256;
+                    l.block = narrow_threads(l.body);
                 } else {
                     unsigned grid = 0, block = 0;
                     if (l.ragged) {

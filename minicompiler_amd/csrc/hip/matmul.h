@@ -132,6 +132,7 @@ enum {
     MCHIP_NARROW_16X64 = 2,         /* 16x64 tiles */
     MCHIP_NARROW_16X32 = 3,         /* 16x32 tiles */
     MCHIP_NARROW_64X64 = 4,         /* 64x64 tiles */
+    MCHIP_NARROW_16X16 = 5,         /* 16x16 tiles, 8 waves, unsplit */
 };
 int mchip_narrow_rows(int shape);
 int mchip_narrow_cols(int shape);
@@ -141,7 +142,9 @@ int mchip_narrow_cols(int shape);
  * tile shape that gives more than half the CUs a tile runs unsplit (the
  * first of 64x64, 32x64, 16x64, 16x32 that does); otherwise 32x64 tiles (16x64, B streamed, for m <= 16)
  * with K cut into *splits ranges of *k_split (a multiple of 16), at most
- * max_splits of them, so that tiles x ranges stays within the CUs. Its
+ * max_splits of them, so that tiles x ranges stays within the CUs; where
+ * that is several ranges, K is at most 1024 (2048 for m = 1) and 16x16
+ * tiles number at most one per CU, those run unsplit instead. Its
  * accumulation order is its own (16x16x4 MFMAs, K pieces per wave added
  * in wave order, then the ranges in range order), not the ring body's.
  * Returns 1 and fills *shape (MCHIP_NARROW_*), *splits and *k_split when

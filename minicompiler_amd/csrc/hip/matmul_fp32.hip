@@ -276,6 +276,7 @@ int launch_narrow(const float* a, const float* b, float* c, int m, int n, int k,
         case MCHIP_NARROW_16X64: narrow_kernel<McNarrow16x64>(a, b, c, m, n, k, s, k_split, depth, part, ctr, ragged); break;
         case MCHIP_NARROW_16X32: narrow_kernel<McNarrow16x32>(a, b, c, m, n, k, s, k_split, depth, part, ctr, ragged); break;
         case MCHIP_NARROW_64X64: narrow_kernel<McNarrow64>(a, b, c, m, n, k, s, k_split, depth, part, ctr, ragged); break;
+        case MCHIP_NARROW_16X16: narrow_kernel<McNarrow16x16>(a, b, c, m, n, k, s, k_split, depth, part, ctr, ragged); break;
         default: return hipErrorInvalidValue;
     }
     const hipError_t e = hipGetLastError();
@@ -514,7 +515,7 @@ extern "C" int mchip_narrow_rows(int shape) {
 }
 
 extern "C" int mchip_narrow_cols(int shape) {
-    return shape == MCHIP_NARROW_16X32 ? 32 : 64;
+    return shape == MCHIP_NARROW_16X16 ? 16 : shape == MCHIP_NARROW_16X32 ? 32 : 64;
 }
 
 extern "C" int mchip_f32_narrow_plan(int m, int n, int k, int max_splits, int cu_count, int force, int* shape,
@@ -579,6 +580,19 @@ extern "C" int mchip_f32_narrow_plan(int m, int n, int k, int max_splits, int cu
     // the CUs and each range at least 64 deep.
     int s = 1;
     while (s * 2 <= max_splits && tiles * s * 2 <= cu_count && k / (s * 2) >= 64) s *= 2;
+    // Several ranges, and with them a sum launch, only where 16x16 tiles would
+    // not do unsplit: at most one per CU, and K short, since a block reads 128
+    // bytes per k (68 with one row). Graph-timed on an MI355X, against the
+    // ranges and their sum: 1x2048x512 3.65 us against 5.1, 16x4096x1024 6.0
+    // against 7.7, 128x512x512 3.7 against 6.3, 64x1024x1024 5.4 against 7.3,
+    // 1x512x2048 5.9 against 5.8 (and one launch less for the host, 2.6 us), but
+    // 4x512x2048 6.9 against 5.7 and 16x512x2048 8.5 against 6.2.
+    if (!force && s > 1 && tiles_of(MCHIP_NARROW_16X16) <= cu_count && k <= (m == 1 ? 2048 : 1024)) {
+        *shape = MCHIP_NARROW_16X16;
+        *k_split = k;
+        *splits = 1;
+        return 1;
+    }
     const int ks = ((k + s - 1) / s + 15) / 16 * 16;
     *shape = sh;
     *k_split = ks;

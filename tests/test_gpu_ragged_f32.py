@@ -1,5 +1,6 @@
 """The FP32 matrix-core GEMMs on what their exact forms do not take: K not a
-multiple of 32 (16), N not of 4, operands at any float address. Edges of the
+multiple of 32 (16), N not of 4, operands at any float address; and the 16x16
+tiles of short K, exact and ragged. Edges of the
 tiles, of the K steps and of the K ranges, the epilogue at the matrix edge,
 against float64 within the FP32 dot-product bound."""
 
@@ -16,7 +17,8 @@ GUARD = 4096
 DOUBLE_BUFFERED = [(128, 129, 65), (129, 130, 95), (300, 131, 1023), (2100, 2049, 100), (2311, 2050, 127),
                    (257, 4, 64), (130, 5, 70), (64, 300, 129)]
 SPLIT_K = [(1, 5, 17, 1), (16, 1001, 777, 6), (20, 70, 33, 1), (65, 513, 2049, 8), (33, 1030, 1000, 4),
-           (1000, 1001, 1023, 4), (257, 515, 4097, 16), (512, 130, 130, 3), (200, 18, 1000, 15), (7, 6, 100, 4)]
+           (1000, 1001, 1023, 4), (257, 515, 4097, 16), (512, 130, 130, 3), (200, 18, 1000, 15), (7, 6, 100, 4),
+           (1, 2048, 512, 8), (1, 516, 2048, 8), (17, 1000, 1023, 4), (128, 512, 144, 2), (31, 33, 129, 2)]
 
 
 def check(mc, oracle, kernel, m, n, k, splits, offsets):

@@ -23,7 +23,8 @@ def test_the_ragged_ring_runs_one_block_per_tile_and_split(mc, m, n, k, depth, w
 
 
 @pytest.mark.parametrize("m,n,k,splits,want", [
-    (16, 1001, 777, 8, (1, 7, 112)),   # as 16x1004x784
+    (16, 1001, 777, 8, (5, 1, 784)),   # as 16x1004x784
+    (16, 1001, 1300, 8, (1, 8, 176)),
     (256, 513, 2047, 8, (2, 1, 2048)),
     (8, 3, 100, 1, None), (8, 4, 15, 1, None),
 ])
@@ -32,3 +33,16 @@ def test_the_ragged_narrow_plan_is_the_exact_one_rounded_up(mc, m, n, k, splits,
     out = [ctypes.c_int() for _ in range(3)]
     ok = f(m, n, k, splits, 256, *[ctypes.byref(x) for x in out])
     assert (tuple(x.value for x in out) if ok else None) == want
+
+
+@pytest.mark.parametrize("m,n,k,splits,want", [
+    (1, 2048, 512, 8, (5, 1, 512)), (1, 512, 2048, 32, (5, 1, 2048)), (4, 512, 1024, 16, (5, 1, 1024)),
+    (16, 4096, 1024, 4, (5, 1, 1024)), (128, 512, 512, 8, (5, 1, 512)),
+    (16, 4096, 1040, 4, (1, 4, 272)), (2, 512, 2048, 32, (1, 32, 64)),  # K too long
+    (16, 4112, 1024, 4, (1, 2, 512)),     # 257 tiles of 16x16
+    (16, 4096, 1024, 1, (1, 1, 1024)),    # no ranges to avoid
+])
+def test_short_k_products_that_would_split_run_16x16_tiles(mc, m, n, k, splits, want):
+    f = mc.library().mchip_f32_narrow_plan
+    out = [ctypes.c_int() for _ in range(3)]
+    assert f(m, n, k, splits, 256, 0, *[ctypes.byref(x) for x in out]) and tuple(x.value for x in out) == want
