@@ -245,8 +245,8 @@ MC_API int mc_matmul_splits(int kernel, int m, int n, int k, int cu_count);     
 /* The K ranges mc_launch_matmul actually runs when given `splits`
  * (16-byte aligned operands, a workspace). No counterpart in the reference,
  * whose split count is exact: here `splits` (and the workspace sized for it)
- * is an upper bound, and split_k's narrow-tile body runs fewer ranges when
- * fewer fill the GPU (256x256x16384 with 64 splits: 8). 1 for kernels that do
+ * is an upper bound: split_k's narrow-tile body and the tensor-core kernels
+ * run fewer ranges when fewer fill the GPU (256x256x16384 with 64 splits: 8). 1 for kernels that do
  * not split, 0 for invalid sizes. */
 MC_API int mc_matmul_k_ranges(int kernel, int m, int n, int k, int splits);
 MC_API long long mc_matmul_workspace_bytes(int kernel, int m, int n, int splits);   /* matmul_kernels.hpp:27-30 */

@@ -587,6 +587,9 @@ extern "C" int mchip_f32_narrow_plan(int m, int n, int k, int max_splits, int cu
     // against 7.7, 128x512x512 3.7 against 6.3, 64x1024x1024 5.4 against 7.3,
     // 1x512x2048 5.9 against 5.8 (and one launch less for the host, 2.6 us), but
     // 4x512x2048 6.9 against 5.7 and 16x512x2048 8.5 against 6.2.
+    // The price is paid on weights just allocated, whose pages every block
+    // walks down all of K: the one-row MLP (D 512, H 2048) takes 34.3 us on its
+    // first pass against 28.7, and 8.0 against 14.7 on each one after.
     if (!force && s > 1 && tiles_of(MCHIP_NARROW_16X16) <= cu_count && k <= (m == 1 ? 2048 : 1024)) {
         *shape = MCHIP_NARROW_16X16;
         *k_split = k;
