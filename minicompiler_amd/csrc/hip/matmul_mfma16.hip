@@ -128,8 +128,9 @@ __device__ __forceinline__ u16x4 round4(f32x4 v) {
 // registers); kBlocks: blocks per CU the register budget is cut for; kAcc: 1,
 // or 4 accumulators per element that take the 32-wide half steps in turn and
 // are added at the end. Where a caller allows K ranges, the 128x128 kernel ran
-// up to four times the ranges these smaller tiles need to fill the chip; four
-// accumulators keep its number of partial sums, and so its rounding error.
+// all of them, up to eight times what these smaller tiles need to fill the
+// chip; ranges x groups x accumulators keep its number of partial sums, and so
+// its rounding error (launch16 picks the forms).
 template <int kBM_, int kBN_, int kWM_, int kWN_, int kG_, int kAhead_, int kBlocks_, int kAcc_ = 1>
 struct Staged {
     static constexpr int kBM = kBM_, kBN = kBN_, kBK = 64;
@@ -607,9 +608,9 @@ struct StagedPlan {
 };
 
 // 128x128 tiles where they give at least four in five CUs one (the line of
-// split_k_splits, past which a caller has no workspace), else 64x64, or 32x64
-// for at most 32 rows; those in K ranges only where they leave half the CUs
-// idle (graph-timed on an MI355X, bf16 operands: 512x1024x2048, 128 tiles of
+// split_k_splits, past which it asks for no ranges: a caller's own count runs
+// as given), else 64x64, or 32x64 for at most 32 rows; those in K ranges only
+// where they leave half the CUs idle (graph-timed on an MI355X, bf16 operands: 512x1024x2048, 128 tiles of
 // 64x64, 14.9 us in 2 ranges with their sum against 22.1 unsplit; 1000^3, 256
 // tiles, 12.5 us unsplit, where the 128x128 kernel in 4 ranges took 26.5).
 StagedPlan staged_plan(int m, int n, int k, int splits) {
@@ -625,7 +626,8 @@ StagedPlan staged_plan(int m, int n, int k, int splits) {
         p.bn = 64;
     }
     p.tiles = tiles(p.bm, p.bn);
-    const long long want = std::max<long long>(1, std::min<long long>(splits, 2 * p.tiles <= cus ? cus / p.tiles : 1));
+    const long long most = p.bm == 128 ? splits : 2 * p.tiles <= cus ? cus / p.tiles : 1;
+    const long long want = std::max<long long>(1, std::min<long long>(splits, most));
     p.k_split = split_len(k, static_cast<int>(want), 64);
     p.depth = std::max(1, (k + p.k_split - 1) / p.k_split);
     return p;
@@ -654,10 +656,16 @@ int launch16(const void* a, const void* b, float* c, int m, int n, int k, hipStr
     // 100.4 against 114.3; bf16 80.8 against 85.6). Eight waves where the
     // registers allow (bf16: 2048^2 34.7 against 44.3 with four; fp32 4096^2
     // 141.8 on four waves against 154.9).
-    // 64x64 of 16-bit operands: two groups of waves, each taking every other K
-    // step, where there is one tile per CU at most (1024^2 14.6 against 18.0)
-    // and the caller's split count leaves the order of adds open; fp32
-    // operands are bound by the loads themselves and gain nothing.
+    // 64x64, where the caller's split count leaves the order of adds open: two
+    // groups of waves, each taking every other K step, where there is one tile
+    // per CU at most (bf16 1024^2 14.6 against 18.0; fp32 operands 768x768x4096
+    // 35.1 against 39.6, 704x768x1024 12.1 against 12.7). The groups also keep
+    // the error of the ranges asked for, up to seven where one range runs
+    // (fp32 operands, 2-norm, 768x768x4096: 1.37e-7 in 7 ranges, 1.73e-7 with
+    // one group of four accumulators, 1.21e-7 with two). fp32 operands in more
+    // than three ranges keep one group: four accumulators per range are enough
+    // sums, and a range has too few steps for two (256x256x2048 in 16 ranges
+    // 9.5 against 9.9).
     const long long cus = std::max(device_cus(), 1);
     if (p.bm == 128) {
         if constexpr (kF32In) {
@@ -676,9 +684,9 @@ int launch16(const void* a, const void* b, float* c, int m, int n, int k, hipStr
     } else if (p.bm == 64) {
         if (splits <= 1) {
             run(Staged<64, 64, 2, 2, 1, 2, 2>{});
-        } else if (kF32In || p.tiles > cus) {
+        } else if (p.tiles > cus || (kF32In && p.depth > 3)) {
             run(Staged<64, 64, 2, 2, 1, 2, 2, 4>{});
-        } else if constexpr (!kF32In) {
+        } else {
             run(Staged<64, 64, 2, 2, 2, 2, 1, 4>{});
         }
     } else if (splits <= 1) {

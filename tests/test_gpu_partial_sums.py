@@ -1,0 +1,73 @@
+"""Rounding error where the library hands out K ranges: the kernels may run
+fewer ranges than that on smaller tiles, but with no larger an error than the
+ranges would have. The comparison sums each range's product (the operator
+unsplit on that slice of K) in range order in FP32."""
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# The 2-norm error of N independent elements scatters by about 1 / sqrt(2 N): 0.4% at the smallest of these sizes, and
+# the two errors are of the same inputs. 3% leaves room for it.
+SLACK = 1.03
+
+
+def rel(c, exact):
+    return np.linalg.norm(c.astype(np.float64) - exact) / np.linalg.norm(exact)
+
+
+def unsplit(mc, kernel, a, b):
+    m, n = a.shape[0], b.shape[1]
+    da, db = mc.DeviceBuffer.from_array(a), mc.DeviceBuffer.from_array(b)
+    c = mc.DeviceBuffer(4 * m * n)
+    mc.launch_matmul(kernel, da.ptr, db.ptr, c.ptr, m, n, a.shape[1])
+    mc.synchronize()
+    return c.download().reshape(m, n)
+
+
+def in_ranges(mc, kernel, a, b, splits, step=64):
+    k = a.shape[1]
+    length = -(-(-(-k // splits)) // step) * step
+    total = None
+    for k0 in range(0, k, length):
+        part = unsplit(mc, kernel, a[:, k0:k0 + length], b[k0:k0 + length])
+        total = part if total is None else total + part
+    return total
+
+
+def rounded(oracle, kernel, x):
+    rnd = oracle.round_bf16 if kernel == "tensor_core_bf16" else oracle.round_f16
+    return rnd(x.reshape(-1)).reshape(x.shape).astype(np.float64)
+
+
+# 36 to 51 tiles of 128x128 (5 to 7 ranges asked for, none run), 13 to 25 (10 to 19 asked for, 2 to 4 run), few rows.
+@pytest.mark.parametrize("kernel", ["tensor_core_bf16", "tensor_core_f16"])
+@pytest.mark.parametrize("m,n,k", [(704, 768, 2048), (640, 832, 4096), (1024, 768, 4095), (640, 640, 4096),
+                                   (1664, 128, 4096), (32, 2048, 4096)])
+def test_the_operator_keeps_the_error_of_the_ranges_it_was_asked_for(device, mc, oracle, kernel, m, n, k):
+    a = oracle.uniform(m * k, 7, -1.0, 1.0).reshape(m, k)
+    b = oracle.uniform(k * n, 8, -1.0, 1.0).reshape(k, n)
+    splits = mc.matmul_splits(kernel, m, n, k, device["cu_count"])
+    da, db, c = mc.DeviceBuffer.from_array(a), mc.DeviceBuffer.from_array(b), mc.DeviceBuffer(4 * m * n)
+    ws = mc.DeviceBuffer(mc.matmul_workspace_bytes(kernel, m, n, splits))
+    print(f"case {kernel} {m}x{n}x{k} splits {splits}", flush=True)
+    mc.launch_matmul(kernel, da.ptr, db.ptr, c.ptr, m, n, k, None, splits, ws.ptr)
+    mc.synchronize()
+    exact = rounded(oracle, kernel, a) @ rounded(oracle, kernel, b)
+    got, want = rel(c.download().reshape(m, n), exact), rel(in_ranges(mc, kernel, a, b, splits), exact)
+    assert splits > 1 and got <= SLACK * want, f"{got:.3e} against {want:.3e} in {splits} ranges"
+
+
+def test_ranges_that_the_library_would_not_ask_for_run_as_given(device, mc, oracle):
+    # 225 tiles of 128x128: the split rule asks for one range; a caller's own count is that of its sums.
+    m, n, k, splits = 1920, 1900, 520, 4
+    a = oracle.uniform(m * k, 7, -1.0, 1.0).reshape(m, k)
+    b = oracle.uniform(k * n, 8, -1.0, 1.0).reshape(k, n)
+    assert mc.matmul_splits("tensor_core_bf16", m, n, k, device["cu_count"]) == 1
+    assert mc.matmul_k_ranges("tensor_core_bf16", m, n, k, splits) == 3
+    da, db, c = mc.DeviceBuffer.from_array(a), mc.DeviceBuffer.from_array(b), mc.DeviceBuffer(4 * m * n)
+    ws = mc.DeviceBuffer(4 * splits * m * n)
+    mc.launch_matmul("tensor_core_bf16", da.ptr, db.ptr, c.ptr, m, n, k, None, splits, ws.ptr)
+    mc.synchronize()
+    assert np.array_equal(c.download().reshape(m, n), in_ranges(mc, "tensor_core_bf16", a, b, splits))
