@@ -31,7 +31,21 @@ struct McFragCfg {
     static constexpr int kThreads = 64 * kW;
     // Steps of 32 k per batch: 10 to 16 loads of 1 KiB.
     static constexpr int kU = kRG + kCG <= 2 ? 8 : kRG + kCG <= 4 ? 4 : 2;
-    // With at most 32 rows one block reads each column of B: streamed.
+    // Accumulators per element, taken by the steps in turn and added at the end.
+    // The operator cuts K into up to 256 / t ranges for t tiles of 128x128, more
+    // than the waves where t is small, which is where the one-fragment-wide tiles
+    // run; with two accumulators their error is no larger for K up to 4096
+    // (2-norm, fp16, 16x2048x4095: 1.28e-7 in 16 ranges, 1.55e-7 with the waves
+    // alone, 1.21e-7 so). Four cost 32 and 64 rows the second block per CU (more
+    // than 128 VGPRs; 32x4096x8000 16.4 us against 15.1). The wider tiles are
+    // picked only for at most as many ranges as they have waves.
+    static constexpr int kAcc = kCG == 1 ? 2 : 1;
+};
+
+// Which of the two register sets a batch is in, as a type.
+template <int kSet>
+struct McFragSet {
+    static constexpr int value = kSet;
 };
 
 template <class Cfg>
@@ -83,11 +97,14 @@ __device__ __forceinline__ void mc_gemm16_frag(const unsigned short* __restrict_
     const int per = (steps + kW - 1) / kW;
     const int s0 = mc_min16(wave * per, steps), s1 = mc_min16(s0 + per, steps);
 
-    mc_f32x4_t acc[kRG][kCG];
+    constexpr int kAcc = Cfg::kAcc;
+    mc_f32x4_t part[kAcc][kRG][kCG];
 #pragma unroll
-    for (int r = 0; r < kRG; ++r)
+    for (int x = 0; x < kAcc; ++x)
 #pragma unroll
-        for (int g = 0; g < kCG; ++g) acc[r][g] = mc_f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int r = 0; r < kRG; ++r)
+#pragma unroll
+            for (int g = 0; g < kCG; ++g) part[x][r][g] = mc_f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
     // The loads of the batch from step s (steps past the wave's last load the
     // last again: a load under a condition would make the compiler wait for
     // every load in flight), then nothing else (a scheduling barrier).
@@ -104,21 +121,22 @@ __device__ __forceinline__ void mc_gemm16_frag(const unsigned short* __restrict_
     };
     // B as the first operand: C^T fragments, so a lane holds four
     // consecutive columns of one row.
-    auto multiply = [&](const McFragRegs<Cfg>& x, int u) {
+    auto multiply = [&](const McFragRegs<Cfg>& x, int u, auto set) {
+        const int to = (decltype(set)::value * kU + u) % kAcc;  // known once unrolled
 #pragma unroll
         for (int r = 0; r < kRG; ++r)
 #pragma unroll
-            for (int g = 0; g < kCG; ++g) acc[r][g] = mc_mfma16<kBf16>(x.b[u][g], x.a[u][r], acc[r][g]);
+            for (int g = 0; g < kCG; ++g) part[to][r][g] = mc_mfma16<kBf16>(x.b[u][g], x.a[u][r], part[to][r][g]);
     };
-    auto whole = [&](const McFragRegs<Cfg>& x) {
+    auto whole = [&](const McFragRegs<Cfg>& x, auto set) {
 #pragma unroll
-        for (int u = 0; u < kU; ++u) multiply(x, u);
+        for (int u = 0; u < kU; ++u) multiply(x, u, set);
         __builtin_amdgcn_sched_barrier(0);
     };
-    auto last = [&](const McFragRegs<Cfg>& x, int s) {
+    auto last = [&](const McFragRegs<Cfg>& x, int s, auto set) {
 #pragma unroll
         for (int u = 0; u < kU; ++u)
-            if (s + u < s1) multiply(x, u);
+            if (s + u < s1) multiply(x, u, set);
     };
     // Two register sets: the loads of batch i + 1 are issued before the MFMAs
     // of batch i.
@@ -128,19 +146,28 @@ __device__ __forceinline__ void mc_gemm16_frag(const unsigned short* __restrict_
         load(x0, s);
         for (; s + 2 * kU < s1; s += 2 * kU) {
             load(x1, s + kU);
-            whole(x0);
+            whole(x0, McFragSet<0>{});
             load(x0, s + 2 * kU);
-            whole(x1);
+            whole(x1, McFragSet<1>{});
         }
         if (s + kU < s1) {
             load(x1, s + kU);
-            whole(x0);
-            last(x1, s + kU);
+            whole(x0, McFragSet<0>{});
+            last(x1, s + kU, McFragSet<1>{});
         } else {
-            last(x0, s);
+            last(x0, s, McFragSet<0>{});
         }
     }
 
+    mc_f32x4_t(&acc)[kRG][kCG] = part[0];
+#pragma unroll
+    for (int step = 1; step < kAcc; step *= 2)
+#pragma unroll
+        for (int x = 0; x < kAcc; x += 2 * step)
+#pragma unroll
+            for (int r = 0; r < kRG; ++r)
+#pragma unroll
+                for (int g = 0; g < kCG; ++g) part[x][r][g] += part[x + step][r][g];
 #pragma unroll
     for (int r = 0; r < kRG; ++r)
 #pragma unroll

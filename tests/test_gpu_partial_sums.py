@@ -71,3 +71,24 @@ def test_ranges_that_the_library_would_not_ask_for_run_as_given(device, mc, orac
     mc.launch_matmul("tensor_core_bf16", da.ptr, db.ptr, c.ptr, m, n, k, None, splits, ws.ptr)
     mc.synchronize()
     assert np.array_equal(c.download().reshape(m, n), in_ranges(mc, "tensor_core_bf16", a, b, splits))
+
+
+def graph_against_ranges(mc, oracle, device, kernel, m, n, k):
+    """The graph's and the ranges' errors for a constant B whose K the operator would cut (K not a multiple of 64)."""
+    a = oracle.uniform(m * k, 7, -1.0, 1.0).reshape(m, k)
+    b = oracle.uniform(k * n, 8, -1.0, 1.0).reshape(k, n)
+    splits = mc.matmul_splits(kernel, m, n, k, device["cu_count"])
+    assert splits > 1 and k % 64 != 0
+    print(f"case graph {kernel} {m}x{n}x{k} splits {splits}", flush=True)
+    c = mc.Compiled(f"input x : f32[{m}, {k}]\nconst w : f32[{k}, {n}] = uniform(seed=8, lo=-1, hi=1)\n"
+                    "h = matmul x, w\noutput h\n", options={"matmul": kernel})
+    exact = rounded(oracle, kernel, a) @ rounded(oracle, kernel, b)
+    return rel(c.run([a.reshape(-1)])[0].reshape(m, n), exact), rel(in_ranges(mc, kernel, a, b, splits), exact)
+
+
+# Tiles of one fragment's width (16, 32 and 64 rows), K as long as they are used for.
+@pytest.mark.parametrize("kernel", ["tensor_core_bf16", "tensor_core_f16"])
+@pytest.mark.parametrize("m,n,k", [(16, 2048, 4095), (8, 1395, 2279), (32, 3001, 4000), (184, 512, 2205), (384, 512, 4095)])
+def test_graphs_on_small_tiles_keep_the_error_of_the_operators_ranges(device, mc, oracle, kernel, m, n, k):
+    got, want = graph_against_ranges(mc, oracle, device, kernel, m, n, k)
+    assert got <= SLACK * want, f"{got:.3e} against {want:.3e} in ranges"
