@@ -71,10 +71,14 @@ def test_packing_writes_the_layout_and_pads_k_with_zeros(device, mc, oracle, ops
 # more and fewer steps than a block has waves; N odd, N % 4 and N % 8; one and several 256-row bands.
 PRODUCTS = [(1, 1, 1), (16, 16, 64), (17, 33, 65), (5, 250, 31), (63, 70, 1000), (64, 64, 512), (65, 129, 577),
             (300, 259, 96), (257, 255, 2047), (32, 260, 520)]
+# K long enough that every wave of every shape runs its two-batch loop (more than 2 kU steps of 32 k per wave: K past
+# 4096 for 16x16 tiles, 2048 for three-fragment ones), then each way of ending it: one batch left or two, whole or not,
+# and a last wave with fewer steps than the others.
+LONG_PRODUCTS = [(5, 37, 4200), (17, 33, 6400), (33, 70, 8257), (16, 16, 12288), (64, 64, 5000), (7, 100, 6144)]
 
 
 @pytest.mark.parametrize("dtype", [1, 2], ids=["bf16", "f16"])
-@pytest.mark.parametrize("m,n,k", PRODUCTS)
+@pytest.mark.parametrize("m,n,k", PRODUCTS + LONG_PRODUCTS)
 def test_every_tile_shape_is_within_the_accumulation_bound(device, mc, oracle, ops, dtype, m, n, k):
     a, b = oracle.uniform(m * k, 7, -1.0, 1.0), oracle.uniform(k * n, 8, -1.0, 1.0)
     rnd = oracle.round_bf16 if dtype == 1 else oracle.round_f16
