@@ -345,7 +345,7 @@ GemmEpilogueKernel generate_gemm_epilogue_kernel(const FusedProgram& program, st
                    std::to_string(mchip_frag_rows(fixed.frag) / 16) + ", " +
                    std::to_string(mchip_frag_cols(fixed.frag) / 16) + ">>";
         } else if (body == GemmBody::Bf16Packed || body == GemmBody::F16Packed) {
-            call = std::string("mc_gemm16_packed<") + type + ">";
+            call = std::string(fixed.frag == MCHIP_TWO_SUMS ? "mc_gemm16_two_sums<" : "mc_gemm16_packed<") + type + ">";
         } else {
             call = std::string("mc_gemm16_fast<") + type + ", true>";
         }

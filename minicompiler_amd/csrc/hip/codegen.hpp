@@ -166,7 +166,7 @@ inline const char* narrow_config(GemmBody body) {
 struct GemmDims {
     int m = 0, n = 0, k = 0, k_split = 0, depth = 1;
     bool ragged = false;  // the ragged form of a ring or narrow body
-    int frag = 0;  // Bf16Frag, F16Frag: the tile shape (MCHIP_FRAG_*)
+    int frag = 0;  // Bf16Frag, F16Frag: the tile shape (MCHIP_FRAG_*); Bf16Packed, F16Packed: MCHIP_TWO_SUMS or any other
 };
 
 GemmEpilogueKernel generate_gemm_epilogue_kernel(const FusedProgram& program, std::size_t acc_input,

@@ -286,8 +286,10 @@ __device__ __forceinline__ void fast_store(const mc_f32x4_t (&acc)[kRowFrags][kF
     }
 }
 
-// One kRows x 256 tile of C at (row0, col0), all of K.
-template <bool kBf16, int kRows, bool kPackedA, bool kPackedB, typename Epilogue>
+// One kRows x 256 tile of C at (row0, col0), all of K. kTwoSums (128 rows, which
+// leave the registers for it): the products of K's first half (whole 64 k) and
+// of the rest are summed apart and the sums added, the bits of two K ranges.
+template <bool kBf16, int kRows, bool kPackedA, bool kPackedB, bool kTwoSums = false, typename Epilogue>
 __device__ __forceinline__ void fast_tile(MC_LDS unsigned char* lds, const unsigned short* __restrict__ a,
                                           const unsigned short* __restrict__ b, float* __restrict__ c, int m, int n,
                                           int k, int row0, int col0, const Epilogue& epilogue) {
@@ -383,7 +385,7 @@ __device__ __forceinline__ void fast_tile(MC_LDS unsigned char* lds, const unsig
     // the fetch of t+1 and waits for t+1, which the other group reads two
     // phases later; loads into LDS complete in issue order.
     const int last = (steps - 1) * kFBK;
-    for (int t = 0; t < steps; ++t) {
+    auto step = [&](int t) {
         const int fetch_k = mc_min16((t + 3) * kFBK, last);
         fast_memory_phase<kRows, kPackedB>(stage(t), stage(t + 3), L, fetch_k, av, bv);
         __builtin_amdgcn_s_waitcnt(0x0070 | (2 * Sh::kFetch - 2));  // vmcnt(2 kFetch - 2), lgkmcnt(0)
@@ -400,6 +402,29 @@ __device__ __forceinline__ void fast_tile(MC_LDS unsigned char* lds, const unsig
 #pragma unroll
             for (int fj = 0; fj < kFColFrags; ++fj) acc[fi][fj] = mc_mfma16<kBf16>(bv[fj], av[fi], acc[fi][fj]);
         step_barrier();
+    };
+    if constexpr (kTwoSums) {
+        // Not unrolled: where K is a constant the compiler unrolled both loops
+        // whole (16 steps each at K = 1000) and the product took 79 us for 24.
+        const int half = (steps / 2 + 1) / 2 * 2;
+        mc_f32x4_t first[Sh::kRowFrags][kFColFrags];
+#pragma clang loop unroll(disable)
+        for (int t = 0; t < half; ++t) step(t);
+#pragma unroll
+        for (int i = 0; i < Sh::kRowFrags; ++i)
+#pragma unroll
+            for (int j = 0; j < kFColFrags; ++j) {
+                first[i][j] = acc[i][j];
+                acc[i][j] = mc_f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+#pragma clang loop unroll(disable)
+        for (int t = half; t < steps; ++t) step(t);
+#pragma unroll
+        for (int i = 0; i < Sh::kRowFrags; ++i)
+#pragma unroll
+            for (int j = 0; j < kFColFrags; ++j) acc[i][j] = first[i][j] + acc[i][j];
+    } else {
+        for (int t = 0; t < steps; ++t) step(t);
     }
     if (!late) step_barrier();
     __builtin_amdgcn_s_waitcnt(0);
@@ -458,4 +483,22 @@ __device__ __forceinline__ void mc_gemm16_packed(const unsigned short* __restric
                                                  const unsigned short* __restrict__ b, float* __restrict__ c, int m,
                                                  int n, int k, const Epilogue& epilogue) {
     mc_gemm16_tiles<kBf16, true, true>(a, b, c, m, n, k, epilogue);
+}
+
+// Both operands packed, 128x256 tiles (one block each, row by row) and two sums
+// per element, for products that the operator cuts into two K ranges and that
+// the small tiles do not take. One chain over all of K has an error up to 1.48
+// times that of the ranges (2-norm, bf16, K = 4095: 3.74e-7 against 2.52e-7);
+// 64x64 tiles, whose waves are four sums, are 30-50% slower. On an MI355X,
+// 1792x1792, K = 1000 / 2047 / 4000: 23.6 / 34.6 / 55.1 us, 23.3 / 33.9 / 54.8
+// with one chain, 33.2 / 50.8 / 80.3 on 64x64 tiles.
+template <bool kBf16, typename Epilogue>
+__device__ __forceinline__ void mc_gemm16_two_sums(const unsigned short* __restrict__ a,
+                                                   const unsigned short* __restrict__ b, float* __restrict__ c, int m,
+                                                   int n, int k, const Epilogue& epilogue) {
+    __shared__ __attribute__((aligned(1024))) unsigned char smem[kFStages * kFStage];
+    MC_LDS unsigned char* lds = (MC_LDS unsigned char*)(smem);
+    const int tiles_n = (n + kFBN - 1) / kFBN, bid = static_cast<int>(blockIdx.x);
+    fast_tile<kBf16, kFBM / 2, true, true, true>(lds, a, b, c, m, n, k, bid / tiles_n * (kFBM / 2),
+                                                 bid % tiles_n * kFBN, epilogue);
 }

@@ -107,7 +107,7 @@ struct Launch {
     bool lowp = false;
     int dtype = 0;
     int kp = 0;
-    int frag = MCHIP_FRAG_NONE;  // the small-tile shape, or the 256x256 tiles
+    int frag = MCHIP_FRAG_NONE;  // the small-tile shape, MCHIP_TWO_SUMS, or the 256x256 tiles
     void* a16 = nullptr;
     void* b16 = nullptr;
     bool convert_a = false, convert_b = false;
@@ -617,6 +617,7 @@ private:
         const bool constant_b = graph_.node(node.inputs[1]).op == OpKind::Constant;
         if (options_.convert_tensor_core_operands && (bf16 || f16) && mchip_pack16_fits(l->m, l->n, l->k) &&
             (constant_b || mchip_mfma16_fast_fits(l->m, l->n, l->k))) {
+            const bool ranges = l->splits > 1 && !mchip_mfma16_fast_fits(l->m, l->n, l->k);
             l->lowp = true;
             l->splits = 1;
             l->dtype = bf16 ? MCHIP_DTYPE_BF16 : MCHIP_DTYPE_F16;
@@ -625,6 +626,9 @@ private:
             // fed per run the product keeps the operator's order of adds (the
             // same bits as mchip_launch_tensor_core on the fp32 operands).
             if (constant_b) l->frag = mchip_mfma16_packed_plan(l->m, l->n, device_.cu_count);
+            // Sizes that only the operator's K ranges ran before they were
+            // packed keep as many sums (the small tiles' waves are enough).
+            if (ranges && l->frag == MCHIP_FRAG_NONE) l->frag = MCHIP_TWO_SUMS;
             l->convert_a = graph_.node(node.inputs[0]).op != OpKind::Constant;
             l->convert_b = !constant_b;
         }
@@ -637,7 +641,7 @@ private:
     GemmBody fused_body(Launch& l) const {
         if (l.lowp) {
             const bool bf16 = l.dtype == MCHIP_DTYPE_BF16;
-            if (l.frag != MCHIP_FRAG_NONE) return bf16 ? GemmBody::Bf16Frag : GemmBody::F16Frag;
+            if (l.frag >= 0) return bf16 ? GemmBody::Bf16Frag : GemmBody::F16Frag;
             return bf16 ? GemmBody::Bf16Packed : GemmBody::F16Packed;
         }
         if (l.matmul == MatmulKernel::SplitK &&

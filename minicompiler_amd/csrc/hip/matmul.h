@@ -46,9 +46,11 @@ int mchip_launch_matmul_lowp_packed(int kernel, int dtype, const void* a_packed,
  * mchip_pack16_fits: the sizes the kernels' 31-bit offsets allow.
  * mchip_launch_mfma16_packed: the product, on 256x256 tiles
  * (MCHIP_FRAG_NONE) or on the small tiles of gemm_mfma16_frag.h;
- * mchip_mfma16_packed_plan picks between them, mchip_frag_* describe a
- * small tile's launch. */
+ * mchip_mfma16_packed_plan picks between them. MCHIP_TWO_SUMS: for what the
+ * operator would cut into two K ranges, with their bits. mchip_frag_* describe
+ * the launch of a small tile or of MCHIP_TWO_SUMS. */
 enum {
+    MCHIP_TWO_SUMS = -2, /* 128x256 tiles, the two halves of K summed apart */
     MCHIP_FRAG_NONE = -1,
     MCHIP_FRAG_16X16 = 0,
     MCHIP_FRAG_16X32 = 1,

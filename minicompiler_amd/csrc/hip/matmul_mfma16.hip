@@ -434,6 +434,13 @@ __global__ void __launch_bounds__(kFThreads, 1) matmul_mfma16_packed(const unsig
     mc_gemm16_packed<kBf16>(a, b, c, m, n, k, McGemm16Store{});
 }
 
+template <bool kBf16>
+__global__ void __launch_bounds__(kFThreads, 1) matmul_mfma16_two_sums(const unsigned short* __restrict__ a,
+                                                                       const unsigned short* __restrict__ b,
+                                                                       float* __restrict__ c, int m, int n, int k) {
+    mc_gemm16_two_sums<kBf16>(a, b, c, m, n, k, McGemm16Store{});
+}
+
 template <bool kBf16, class Cfg>
 __global__ void __launch_bounds__(Cfg::kThreads) matmul_mfma16_frag(const unsigned short* __restrict__ a,
                                                                     const unsigned short* __restrict__ b,
@@ -854,8 +861,8 @@ extern "C" int mchip_pack16_b_f32(int dtype, const float* b, void* packed, int k
     return hipGetLastError();
 }
 
-extern "C" int mchip_frag_rows(int shape) { return 16 << (shape / 3); }
-extern "C" int mchip_frag_cols(int shape) { return 16 << (shape % 3); }
+extern "C" int mchip_frag_rows(int shape) { return shape == MCHIP_TWO_SUMS ? kFBM / 2 : 16 << (shape / 3); }
+extern "C" int mchip_frag_cols(int shape) { return shape == MCHIP_TWO_SUMS ? kFBN : 16 << (shape % 3); }
 extern "C" int mchip_frag_threads(int shape) { return shape == MCHIP_FRAG_64X64 ? 256 : 512; }
 
 extern "C" unsigned mchip_frag_grid(int shape, int m, int n) {
@@ -900,8 +907,12 @@ int launch_packed(int shape, const unsigned short* a, const unsigned short* b, f
                            dim3(kFThreads), 0, s, a, b, c, m, n, kp);
         return hipGetLastError();
     }
+    if (shape < MCHIP_TWO_SUMS || shape > MCHIP_FRAG_64X64) return hipErrorInvalidValue;
     const unsigned grid = mchip_frag_grid(shape, m, n);
     switch (shape) {
+        case MCHIP_TWO_SUMS:
+            hipLaunchKernelGGL((matmul_mfma16_two_sums<kBf16>), dim3(grid), dim3(kFThreads), 0, s, a, b, c, m, n, kp);
+            return hipGetLastError();
         case MCHIP_FRAG_16X16: return launch_frag<kBf16, 1, 1>(a, b, c, m, n, kp, grid, s);
         case MCHIP_FRAG_16X32: return launch_frag<kBf16, 1, 2>(a, b, c, m, n, kp, grid, s);
         case MCHIP_FRAG_16X64: return launch_frag<kBf16, 1, 4>(a, b, c, m, n, kp, grid, s);

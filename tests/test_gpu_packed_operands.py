@@ -15,6 +15,7 @@ pytestmark = pytest.mark.gpu
 
 SMALL_SHAPES = range(9)  # MCHIP_FRAG_*: 16, 32, 64 rows x 16, 32, 64 columns
 TILES_256 = -1
+TWO_SUMS = -2  # 128x256 tiles, the halves of K summed apart
 GUARD = 4096
 
 
@@ -85,7 +86,7 @@ def test_every_tile_shape_is_within_the_accumulation_bound(device, mc, oracle, o
     exact, absdot = oracle.gemm_f64(rnd(a), rnd(b), m, k, n)
     bound = gamma(k) * absdot + 2 * U32 * np.abs(exact) + 1e-30
     pa, pb = pack(mc, ops, "a", dtype, a, m, k), pack(mc, ops, "b", dtype, b, n, k)
-    for shape in [TILES_256, *SMALL_SHAPES]:
+    for shape in [TWO_SUMS, TILES_256, *SMALL_SHAPES]:
         print(f"case product {m}x{n}x{k} dtype {dtype} shape {shape}", flush=True)
         c = mc.DeviceBuffer.from_array(np.full(m * n + GUARD, np.nan, np.float32))
         assert ops.mchip_launch_mfma16_packed(dtype, shape, pa.ptr, pb.ptr, c.ptr, m, n, k, None) == 0
@@ -101,7 +102,7 @@ def test_infinities_stay_in_their_row_and_column(device, mc, oracle, ops):
     a[3, 0] = np.inf
     b[k - 1, 5] = np.nan
     pa, pb = pack(mc, ops, "a", 1, a.ravel(), m, k), pack(mc, ops, "b", 1, b.ravel(), n, k)
-    for shape in [TILES_256, *SMALL_SHAPES]:
+    for shape in [TWO_SUMS, TILES_256, *SMALL_SHAPES]:
         c = mc.DeviceBuffer(m * n * 4)
         assert ops.mchip_launch_mfma16_packed(1, shape, pa.ptr, pb.ptr, c.ptr, m, n, k, None) == 0
         mc.synchronize()

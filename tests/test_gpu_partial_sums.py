@@ -92,3 +92,20 @@ def graph_against_ranges(mc, oracle, device, kernel, m, n, k):
 def test_graphs_on_small_tiles_keep_the_error_of_the_operators_ranges(device, mc, oracle, kernel, m, n, k):
     got, want = graph_against_ranges(mc, oracle, device, kernel, m, n, k)
     assert got <= SLACK * want, f"{got:.3e} against {want:.3e} in ranges"
+
+
+# 193 to 204 tiles of 128x128: past the small tiles' line, and still two ranges. K on and off 128, one row and one column
+# of a tile; a fused group must not change the product.
+@pytest.mark.parametrize("kernel", ["tensor_core_bf16", "tensor_core_f16"])
+@pytest.mark.parametrize("m,n,k", [(1792, 1792, 1000), (1660, 1909, 1025), (65, 25500, 2047), (3584, 896, 200)])
+def test_graphs_past_the_small_tiles_have_the_bits_of_the_operators_two_ranges(device, mc, oracle, kernel, m, n, k):
+    a = oracle.uniform(m * k, 7, -1.0, 1.0).reshape(m, k)
+    b = oracle.uniform(k * n, 8, -1.0, 1.0).reshape(k, n)
+    assert mc.matmul_splits(kernel, m, n, k, device["cu_count"]) == 2
+    want = in_ranges(mc, kernel, a, b, 2).reshape(-1)
+    text = (f"input x : f32[{m}, {k}]\nconst w : f32[{k}, {n}] = uniform(seed=8, lo=-1, hi=1)\nh = matmul x, w\n")
+    for tail, ref in (("output h\n", want), ("y = neg h\nz = relu y\noutput z\n", np.maximum(-want, 0))):
+        print(f"case two sums {kernel} {m}x{n}x{k} {tail!r}", flush=True)
+        c = mc.Compiled(text + tail, options={"matmul": kernel})
+        assert len(c.launch_nodes) == 1
+        assert np.array_equal(c.run([a.reshape(-1)])[0], ref)
