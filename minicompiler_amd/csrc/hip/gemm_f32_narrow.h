@@ -220,8 +220,11 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
     // many partial sums the rounding error is no larger. Relative error in
     // the 2-norm and time on an MI355X, the two-stage body / one accumulator
     // / these: 449x1263x1472 2.9e-7 39.1 us / 3.5e-7 29.0 us / 2.5e-7 30.6 us,
-    // 64x2032x1327 1.9e-7 19.0 us / 3.3e-7 8.7 us / 1.7e-7 8.7 us.
-    constexpr int kAcc = Cfg::kAcc > 1 || !kRagged ? Cfg::kAcc : kRG * kVec <= 8 ? 4 : 2;
+    // 64x2032x1327 1.9e-7 19.0 us / 3.3e-7 8.7 us / 1.7e-7 8.7 us. 16x32 tiles
+    // take over from the most ranges and keep eight (256x261x2047, 22 ranges
+    // before: 1.97e-7, 2.11e-7 with four, 1.57e-7 with eight).
+    constexpr int kAcc =
+        Cfg::kAcc > 1 || !kRagged ? Cfg::kAcc : kRG * kVec <= 2 ? 8 : kRG * kVec <= 8 ? 4 : 2;
     mc_nw_f32x4 part_acc[kAcc][kRG][kVec] = {};
     // Loads of `units` groups from group g into x, then (after a scheduling
     // barrier: left to itself the scheduler interleaves each load with the

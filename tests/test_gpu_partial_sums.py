@@ -109,3 +109,20 @@ def test_graphs_past_the_small_tiles_have_the_bits_of_the_operators_two_ranges(d
         c = mc.Compiled(text + tail, options={"matmul": kernel})
         assert len(c.launch_nodes) == 1
         assert np.array_equal(c.run([a.reshape(-1)])[0], ref)
+
+
+# FP32, N or K off the exact forms' steps, on the narrow tiles of each width that run one range where many are asked for.
+@pytest.mark.parametrize("m,n,k", [(256, 261, 2047), (250, 300, 1700), (512, 261, 2047), (1000, 1001, 1023), (64, 2032, 1327)])
+def test_ragged_fp32_products_keep_the_error_of_the_ranges_they_were_asked_for(device, mc, oracle, m, n, k):
+    a = oracle.uniform(m * k, 7, -1.0, 1.0).reshape(m, k)
+    b = oracle.uniform(k * n, 8, -1.0, 1.0).reshape(k, n)
+    splits = mc.matmul_splits("split_k", m, n, k, device["cu_count"])
+    da, db, c = mc.DeviceBuffer.from_array(a), mc.DeviceBuffer.from_array(b), mc.DeviceBuffer(4 * m * n)
+    ws = mc.DeviceBuffer(mc.matmul_workspace_bytes("split_k", m, n, splits))
+    print(f"case ragged fp32 {m}x{n}x{k} splits {splits}", flush=True)
+    mc.launch_matmul("split_k", da.ptr, db.ptr, c.ptr, m, n, k, None, splits, ws.ptr)
+    mc.synchronize()
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    got = rel(c.download().reshape(m, n), exact)
+    want = rel(in_ranges(mc, "double_buffered", a, b, splits, step=32), exact)
+    assert splits > 1 and got <= SLACK * want, f"{got:.3e} against {want:.3e} in {splits} ranges"
