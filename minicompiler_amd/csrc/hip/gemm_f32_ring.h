@@ -15,9 +15,9 @@
 // Requirements (checked by the host): K (and the split size) a multiple of
 // 32, N a multiple of 4, A, B, C and the partials 16-byte aligned, every
 // split non-empty; counters (when given): one zeroed unsigned per tile.
-// Rows past M and columns past N are clamped to the last row / column
-// chunk, so every load is in bounds; what they bring only reaches C elements
-// that are not stored.
+// Rows past M read the last row and columns past N the tile's first chunk, so
+// every load is in bounds; what they bring only reaches C elements that are
+// not stored.
 //
 // The ragged form (kRagged, staged configurations) takes any K of 64 or more,
 // any N of 4 or more and any float-aligned operands, one unit per block, no
@@ -622,8 +622,9 @@ __device__ __forceinline__ void mc_gemm_f32_ring(const float* __restrict__ a, co
     // bb 1024 / kBRow + l / (kBRow / 16), physical chunk l % (kBRow / 16),
     // logical chunk that ^ 8 (k row / 16 % 2).
     constexpr int kLanesPerBRow = Cfg::kBRow / 16;
-    // Offsets are from the unit's origin; clamped rows and columns are at or
-    // past it (row0 <= m - 1, col0 <= n - 4).
+    // Offsets are from the unit's origin. Rows past M read row M - 1, columns past
+    // N the tile's first chunk: both at or past the origin, also where N is no
+    // multiple of 4 and a last tile has fewer than 4 columns.
     auto fetch_of = [&](const McRingUnit& u) {
         McRingFetch<Cfg> f;
         f.a_rsrc = mc_ring_rsrc(a + static_cast<long long>(u.row0) * k + u.kb);
@@ -640,7 +641,7 @@ __device__ __forceinline__ void mc_gemm_f32_ring(const float* __restrict__ a, co
             const int kk = (Cfg::kFB * wave + i) * (1024 / Cfg::kBRow) + lane / kLanesPerBRow;
             const int g = (lane % kLanesPerBRow) ^ (8 * ((kk >> 4) & 1));
             int col = u.col0 + 4 * g;
-            if (kRagged ? col >= n : col > n - 4) col = n - 4;
+            if (col >= n) col = u.col0;
             f.b_off[i] = 4 * (kk * n + col - u.col0);
         }
         f.b_step = 4 * Cfg::kBK * n;
