@@ -320,7 +320,11 @@ MfmaPlan plan_mfma_f32(bool double_buffer, bool a16, bool b16, bool c16, bool ws
             p.shape = shape;
             p.k_split = nk;
             p.depth = ns;
-            if (ns > 1 && !has_ws) p.status = hipErrorInvalidValue;  // as the ring would
+            // Several ranges need a workspace, as on the ring; so do those asked
+            // for where the 16x16 tiles or a ragged form run one instead.
+            const int asked = split_len(k, splits, kMBK);
+            const bool ranges = ns > 1 || shape == MCHIP_NARROW_16X16 || (p.ragged && (k + asked - 1) / asked > 1);
+            if (ranges && !has_ws) p.status = hipErrorInvalidValue;
             return p;
         }
     }

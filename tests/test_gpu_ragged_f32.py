@@ -89,3 +89,20 @@ def test_fused_groups_at_the_matrix_edge(device, mc, oracle, m, n, k, matmul):
     assert len(c.launch_nodes) == 1 and len(c.launch_nodes[0]) == 2
     got = run_into_prefilled(mc, c, [x, w, b, r])[0].astype(np.float64)
     assert np.all(np.abs(got - want) <= fp32_gemm_bound(exact, absdot, k) + 4 * 2.0 ** -24 * (np.abs(exact) + 2.0))
+
+
+# 16x16 tiles (exact and ragged), ragged narrow tiles unsplit, the ragged ring; last, products of one range, which need
+# no workspace, whatever is asked for.
+@pytest.mark.parametrize("m,n,k,splits,offset,refused", [
+    (16, 512, 1024, 4, 0, True), (1, 2048, 512, 8, 0, True), (17, 1000, 1023, 4, 0, True), (300, 260, 100, 2, 0, True),
+    (256, 517, 2047, 8, 0, True), (256, 512, 2048, 8, 4, True), (1300, 1301, 1500, 2, 0, True),
+    (256, 512, 2048, 8, 0, False), (300, 260, 30, 4, 0, False), (300, 260, 100, 1, 0, False)])
+def test_ranges_without_a_workspace_are_refused_whatever_number_of_them_runs(device, mc, m, n, k, splits, offset, refused):
+    a, b, c = (mc.DeviceBuffer(4 * x + 16) for x in (m * k, k * n, m * n))
+    run = lambda: mc.launch_matmul("split_k", a.ptr + offset, b.ptr, c.ptr, m, n, k, None, splits, None)
+    if refused:
+        with pytest.raises(mc.HipError):
+            run()
+    else:
+        run()
+    mc.synchronize()
