@@ -145,7 +145,7 @@ int mchip_narrow_cols(int shape);
  * first of 64x64, 32x64, 16x64, 16x32 that does); otherwise 32x64 tiles (16x64, B streamed, for m <= 16)
  * with K cut into *splits ranges of *k_split (a multiple of 16), at most
  * max_splits of them, so that tiles x ranges stays within the CUs; where
- * that is several ranges, K is at most 1024 (2048 for m = 1) and 16x16
+ * that is several ranges, K is at most 1024 and 16x16
  * tiles number at most one per CU, those run unsplit instead. Its
  * accumulation order is its own (16x16x4 MFMAs, K pieces per wave added
  * in wave order, then the ranges in range order), not the ring body's.

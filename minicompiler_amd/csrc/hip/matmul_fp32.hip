@@ -585,16 +585,24 @@ extern "C" int mchip_f32_narrow_plan(int m, int n, int k, int max_splits, int cu
     int s = 1;
     while (s * 2 <= max_splits && tiles * s * 2 <= cu_count && k / (s * 2) >= 64) s *= 2;
     // Several ranges, and with them a sum launch, only where 16x16 tiles would
-    // not do unsplit: at most one per CU, and K short, since a block reads 128
-    // bytes per k (68 with one row). Graph-timed on an MI355X, against the
-    // ranges and their sum: 1x2048x512 3.65 us against 5.1, 16x4096x1024 6.0
-    // against 7.7, 128x512x512 3.7 against 6.3, 64x1024x1024 5.4 against 7.3,
-    // 1x512x2048 5.9 against 5.8 (and one launch less for the host, 2.6 us), but
-    // 4x512x2048 6.9 against 5.7 and 16x512x2048 8.5 against 6.2.
-    // The price is paid on weights just allocated, whose pages every block
-    // walks down all of K: the one-row MLP (D 512, H 2048) takes 34.3 us on its
-    // first pass against 28.7, and 8.0 against 14.7 on each one after.
-    if (!force && s > 1 && tiles_of(MCHIP_NARROW_16X16) <= cu_count && k <= (m == 1 ? 2048 : 1024)) {
+    // not do unsplit: at most one per CU, and K short, since every block walks
+    // down all of K. Graph-timed on an MI355X against the ranges and their sum,
+    // one weight matrix / matrices past the 256 MB MALL, us:
+    //   m x n x k         ranges       16x16
+    //   1 x 2048 x 512    4.6 / 5.1    3.0 / 4.8
+    //   16 x 2048 x 512   5.2 / 5.7    3.3 / 5.5
+    //   128 x 512 x 512   6.0 / 6.4    3.4 / 4.0
+    //   1 x 2048 x 1024   4.8 / 5.8    3.6 / 6.7
+    //   16 x 2048 x 1024  5.4 / 6.3    4.4 / 8.1
+    //   64 x 1024 x 1024  6.6 / 7.6    4.7 / 7.2
+    //   1 x 2048 x 1536   5.1 / 6.4    4.2 / 8.4
+    //   1 x 512 x 2048    4.9 / 5.6    4.6 / 10.0
+    //   4 x 512 x 2048    5.0 / 5.8    4.7 / 10.5
+    //   16 x 512 x 2048   5.5 / 6.1    6.4 / 12.9
+    // (2, 3 and 4 rows are as 1.) From the host a launch less is worth another
+    // 2.6 us. Up to K = 1024 the first call on a new matrix is no slower either
+    // (1x512x1024 7.0 us against 8.1); at 2048 it is (9.2 against 8.7).
+    if (!force && s > 1 && tiles_of(MCHIP_NARROW_16X16) <= cu_count && k <= 1024) {
         *shape = MCHIP_NARROW_16X16;
         *k_split = k;
         *splits = 1;

@@ -36,9 +36,9 @@ def test_the_ragged_narrow_plan_is_the_exact_one_rounded_up(mc, m, n, k, splits,
 
 
 @pytest.mark.parametrize("m,n,k,splits,want", [
-    (1, 2048, 512, 8, (5, 1, 512)), (1, 512, 2048, 32, (5, 1, 2048)), (4, 512, 1024, 16, (5, 1, 1024)),
+    (1, 2048, 512, 8, (5, 1, 512)), (4, 512, 1024, 16, (5, 1, 1024)),
     (16, 4096, 1024, 4, (5, 1, 1024)), (128, 512, 512, 8, (5, 1, 512)),
-    (16, 4096, 1040, 4, (1, 4, 272)), (2, 512, 2048, 32, (1, 32, 64)),  # K too long
+    (16, 4096, 1040, 4, (1, 4, 272)), (1, 512, 2048, 32, (1, 32, 64)), (2, 512, 2048, 32, (1, 32, 64)),  # K too long
     (16, 4112, 1024, 4, (1, 2, 512)),     # 257 tiles of 16x16
     (16, 4096, 1024, 1, (1, 1, 1024)),    # no ranges to avoid
 ])
