@@ -168,12 +168,14 @@ MC_API int mc_generate_elementwise_kernel(const char* program, const char* input
                                           int size);
 /* The matrix-core GEMM whose store applies `program` (its input
  * `acc_input` is the accumulated value; the others are read by access class
- * against `out_shape`), as the executable generates it for a matmul with a
- * fused elementwise consumer, on GEMM body `body`: "two_stage" (or NULL),
+ * against `out_shape`), for a matmul with a fused elementwise consumer, on
+ * GEMM body `body`: "two_stage" (or NULL),
  * "ring_big", "ring_wide", "ring_wide8", "ring_mid", "ring_thin", "narrow16",
  * "narrow32", "narrow16x64", "narrow16x32", "narrow64", "narrow16x16",
- * "bf16", "f16" (A packed), "bf16_packed", "f16_packed" (both operands packed), "bf16_frag",
- * "f16_frag" (both packed, small tiles). Works without a device. */
+ * "bf16_packed", "f16_packed" (both operands packed), "bf16_frag", "f16_frag"
+ * (both packed, small tiles), as the executable generates it; and "bf16",
+ * "f16" (A packed, B row-major), which no executable uses. Works without a
+ * device. */
 MC_API int mc_generate_gemm_epilogue_kernel(const char* program, int acc_input, const char* input_shapes,
                                             const char* out_shape, int vectorized_operands, const char* body,
                                             char* out, int size);
@@ -246,8 +248,10 @@ MC_API int mc_matmul_splits(int kernel, int m, int n, int k, int cu_count);     
  * (16-byte aligned operands, a workspace). No counterpart in the reference,
  * whose split count is exact: here `splits` (and the workspace sized for it)
  * is an upper bound: split_k's narrow-tile body and the tensor-core kernels
- * run fewer ranges when fewer fill the GPU (256x256x16384 with 64 splits: 8). 1 for kernels that do
- * not split, 0 for invalid sizes. */
+ * run fewer ranges when fewer fill the GPU (256x256x16384 with 64 splits: 8).
+ * Pass the workspace whenever several are asked for: most products are
+ * refused without it, also where one range runs. 1 for kernels that do not
+ * split, 0 for invalid sizes. */
 MC_API int mc_matmul_k_ranges(int kernel, int m, int n, int k, int splits);
 MC_API long long mc_matmul_workspace_bytes(int kernel, int m, int n, int splits);   /* matmul_kernels.hpp:27-30 */
 MC_API int mc_resolve_matmul_kernel(int kernel, int m, int n, int k, int cu_count); /* cuda_backend.hpp:45-49 */

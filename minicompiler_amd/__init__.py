@@ -674,7 +674,7 @@ def matmul_splits(kernel: int | str, m: int, n: int, k: int, cu_count: int) -> i
 
 def matmul_k_ranges(kernel: int | str, m: int, n: int, k: int, splits: int) -> int:
     """The K ranges launch_matmul runs given `splits` (an upper bound: the
-    narrow-tile body of split_k may run fewer)."""
+    narrow-tile body of split_k and the tensor-core kernels may run fewer)."""
     return int(library().mc_matmul_k_ranges(matmul_kernel_id(kernel), m, n, k, splits))
 
 

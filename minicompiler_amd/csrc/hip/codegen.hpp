@@ -100,9 +100,9 @@ enum class GemmBody {
     F32Narrow16x32,  // likewise, 16x32 tiles
     F32Narrow64,  // likewise, 64x64 tiles
     F32Narrow16x16,  // likewise, 16x16 tiles, 8 waves (short K, few tiles)
-    Bf16Fast,     // bf16 operands in HBM, 256x256 tiles, 512 lanes, one block per tile
-    F16Fast,      // fp16 operands, likewise
-    Bf16Packed,   // bf16, the same tiles, both operands packed
+    Bf16Fast,     // bf16 operands in HBM, A packed, 256x256 tiles, 512 lanes, one block per tile
+    F16Fast,      // fp16 operands, likewise (both for the source-dump call only)
+    Bf16Packed,   // bf16, the same tiles (or MCHIP_TWO_SUMS), both operands packed
     F16Packed,    // fp16, likewise
     Bf16Frag,     // bf16, both operands packed, 16x16 to 64x64 tiles (gemm_mfma16_frag.h)
     F16Frag,      // fp16, likewise
@@ -156,7 +156,8 @@ inline const char* narrow_config(GemmBody body) {
 // launch adds the partials itself and the sum kernel is not launched; the
 // two-stage body ignores counters. 16-bit bodies (one block of 512 lanes per
 // 256x256 tile, or the grid and block of mchip_frag_grid / _threads):
-// (a, b, c, m, n, k, epi), k the padded K where both operands are packed. epi holds one float pointer per program
+// (a, b, c, m, n, k, epi), k the padded K where both operands are packed.
+// epi holds one float pointer per program
 // input (that of `acc_input` unused). `vectorized_operands` (FP32): A and B
 // rows allow 16-byte loads (k and n multiples of 4, 16-byte aligned).
 // The product's dimensions, when the kernel serves one shape only: the
@@ -166,7 +167,9 @@ inline const char* narrow_config(GemmBody body) {
 struct GemmDims {
     int m = 0, n = 0, k = 0, k_split = 0, depth = 1;
     bool ragged = false;  // the ragged form of a ring or narrow body
-    int frag = 0;  // Bf16Frag, F16Frag: the tile shape (MCHIP_FRAG_*); Bf16Packed, F16Packed: MCHIP_TWO_SUMS or any other
+    // Bf16Frag, F16Frag: the tile shape (MCHIP_FRAG_*). Bf16Packed, F16Packed:
+    // MCHIP_TWO_SUMS, or any other value for the 256x256 tiles.
+    int frag = 0;
 };
 
 GemmEpilogueKernel generate_gemm_epilogue_kernel(const FusedProgram& program, std::size_t acc_input,

@@ -113,14 +113,15 @@ using McNarrow16x32 = McNarrowCfg<1, 2, 4, 2, false>;
 // 31-36 us against 22.5 us for one block per CU in two rounds.
 using McNarrow64 = McNarrowCfg<4, 4, 4, 2, false, 96>;
 // 16x16 tiles, eight waves: for products that any other shape would have to
-// split over K ranges, and K short enough that a block's 128 bytes per k (16
-// rows of A, 16 columns of B, at about 45 GB/s per CU) cost less than the
-// ranges' sum launch (mchip_f32_narrow_plan). Eight accumulators per element:
-// a wave's chain of adds is as short as with the ranges, and the error no
-// larger (relative in the 2-norm, ranges / four accumulators / eight:
-// 1x512x2048 1.37e-7 / 1.58e-7 / 1.22e-7, 16x4096x1024 1.55e-7 / 1.20e-7 /
-// 1.00e-7). Batches of one group: 2, 4 and 8 groups were no faster
-// (1x512x2048 5.9 us against 6.1, 6.2 and 6.7).
+// split over K ranges, and K short enough that a block's way down all of K
+// (16 rows of A and 16 columns of B: 128 bytes per k) costs less than the
+// ranges' sum launch (mchip_f32_narrow_plan has the figures). Eight accumulators
+// per element: a wave's chain of adds is as short as with the ranges, and the
+// error no larger (relative in the 2-norm, ranges / four accumulators / eight:
+// 16x4096x1024 1.55e-7 / 1.20e-7 / 1.00e-7). Batches of one group: 2, 4 and 8
+// groups were no faster (1x2048x1024 on an MI355X, graph-timed, one matrix /
+// matrices past the MALL: 3.7 / 6.6 us against 3.7 / 6.9, 4.1 / 6.9 and
+// 4.4 / 7.6).
 using McNarrow16x16 = McNarrowCfg<1, 1, 8, 1, false, 16, 8>;
 
 // A 16-, 8- or 4-byte buffer load at (voffset + soffset) from the resource's

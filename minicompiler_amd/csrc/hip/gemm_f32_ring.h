@@ -10,7 +10,8 @@
 // is accumulated by the same v_mfma_f32_32x32x2_f32 sequence (the 32-wide K
 // step split into k and k + 16 slot pairs, four k per LDS read), so every
 // configuration here and that body give identical bits, and any of them may
-// serve a request they all accept.
+// serve a request they all accept. (The ragged form, below, adds the end of K
+// first, where it loads that apart.)
 //
 // Requirements (checked by the host): K (and the split size) a multiple of
 // 32, N a multiple of 4, A, B, C and the partials 16-byte aligned, every
@@ -27,9 +28,8 @@
 // care: the unit that holds it loads its last K % 32 rows (32 when N alone is
 // ragged) float by float with zeros past K, in the prologue, as its first
 // step, so its latency is the first load's that every unit waits for anyway.
-// The order of the other steps is unchanged. On an MI355X, 2000x1001x1023 + bias
-// + ReLU 99.2 us on the two-stage body, 44.8 so (64x64 narrow tiles), and
-// 3810x1960x744 on this body 93.5 against 111.3.
+// The order of the other steps is unchanged. On an MI355X 3810x1960x744 took
+// 111.3 us on the two-stage body and 93.5 so.
 #pragma once
 
 typedef float mc_ring_f32x4 __attribute__((ext_vector_type(4)));

@@ -586,22 +586,23 @@ extern "C" int mchip_f32_narrow_plan(int m, int n, int k, int max_splits, int cu
     while (s * 2 <= max_splits && tiles * s * 2 <= cu_count && k / (s * 2) >= 64) s *= 2;
     // Several ranges, and with them a sum launch, only where 16x16 tiles would
     // not do unsplit: at most one per CU, and K short, since every block walks
-    // down all of K. Graph-timed on an MI355X against the ranges and their sum,
-    // one weight matrix / matrices past the 256 MB MALL, us:
+    // down all of K. The gain is the sum's launch, the price is paid on weights
+    // that no cache holds. On an MI355X against the ranges and their sum, us:
+    // graph-timed on one weight matrix / per call for twelve matrices in a row
+    // that no cache holds, launched from the host.
     //   m x n x k         ranges       16x16
-    //   1 x 2048 x 512    4.6 / 5.1    3.0 / 4.8
-    //   16 x 2048 x 512   5.2 / 5.7    3.3 / 5.5
-    //   128 x 512 x 512   6.0 / 6.4    3.4 / 4.0
-    //   1 x 2048 x 1024   4.8 / 5.8    3.6 / 6.7
-    //   16 x 2048 x 1024  5.4 / 6.3    4.4 / 8.1
-    //   64 x 1024 x 1024  6.6 / 7.6    4.7 / 7.2
-    //   1 x 2048 x 1536   5.1 / 6.4    4.2 / 8.4
-    //   1 x 512 x 2048    4.9 / 5.6    4.6 / 10.0
-    //   4 x 512 x 2048    5.0 / 5.8    4.7 / 10.5
-    //   16 x 512 x 2048   5.5 / 6.1    6.4 / 12.9
-    // (2, 3 and 4 rows are as 1.) From the host a launch less is worth another
-    // 2.6 us. Up to K = 1024 the first call on a new matrix is no slower either
-    // (1x512x1024 7.0 us against 8.1); at 2048 it is (9.2 against 8.7).
+    //   1 x 2048 x 512    4.6 / 8.0    3.0 / 5.3
+    //   16 x 2048 x 512   5.2 / 7.9    3.3 / 5.9
+    //   64 x 1024 x 512   6.1 / 8.2    3.4 / 5.3
+    //   1 x 2048 x 1024   4.8 / 7.9    3.6 / 7.4
+    //   16 x 2048 x 1024  5.4 / 8.2    4.4 / 8.9
+    //   64 x 1024 x 1024  6.6 / 8.4    4.7 / 8.0
+    //   1 x 2048 x 1536   5.1 / 8.1    4.2 / 9.9
+    //   1 x 512 x 2048    4.9 / 7.9    4.6 / 11.0
+    //   4 x 512 x 2048    5.0 / 8.0    4.7 / 11.3
+    //   16 x 512 x 2048   5.5 / 8.1    6.4 / 13.6
+    // (2 and 3 rows are as 1 and 4.) Where the two meet, at K = 1024, one call
+    // alone on such weights takes 9.6 us against 8.5 (1 x 2048).
     if (!force && s > 1 && tiles_of(MCHIP_NARROW_16X16) <= cu_count && k <= 1024) {
         *shape = MCHIP_NARROW_16X16;
         *k_split = k;

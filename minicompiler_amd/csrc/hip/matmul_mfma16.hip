@@ -12,11 +12,14 @@
 //                          LDS) or 16-bit, any shape and alignment, split K;
 //   matmul_mfma16_fast     16-bit operands, B row-major, 256x256 tiles
 //                          (gemm_mfma16_fast.h);
-//   matmul_mfma16_packed, matmul_mfma16_frag   both operands packed
-//                          (gemm_mfma16_fast.h, gemm_mfma16_frag.h).
-// Every kernel that does not split K adds each element's products in the same
-// order (32 k per MFMA, K ascending), so they give the same bits, except the
-// frag kernels, which split K over a block's waves.
+//   matmul_mfma16_packed, matmul_mfma16_two_sums, matmul_mfma16_frag   both
+//                          operands packed (gemm_mfma16_fast.h, _frag.h).
+// Asked for one K range, the staged and fast kernels add each element's products
+// in one order (32 k per MFMA, K ascending) and give the same bits, and so does
+// the packed one; two_sums has the bits of two such ranges added. The others
+// have orders of their own: the frag kernels (a block's waves and accumulators)
+// and the staged kernel asked for several ranges (wave groups and accumulators,
+// whatever number of ranges runs).
 //
 // v_mfma_f32_16x16x32_*: lane l supplies row (A) / column (B) l % 16 and
 // eight k values from group l / 16; A and B use the same k assignment, so
@@ -96,16 +99,19 @@ __device__ __forceinline__ u16x4 round4(f32x4 v) {
 // ---------------------------------------------------------------- staged
 //
 // Row-major A [m, k] and B [k, n] of fp32 or 16-bit elements at any element
-// address. What bounds it: at fp32 operands the CU's vector-memory path (a
-// 128x128x64 step loads 64 KiB for 512 cycles of MFMA); at small products the
-// latency of each step's loads.
+// address. What bounds it is each K step's chain of load, rounding, LDS write and
+// barrier, with one block per CU. Counters on an MI355X: 2048^3 from fp32 keeps
+// the matrix units 21% busy and brings each CU 67 GB/s from its L2 (81% hits), the
+// waves 29% waiting, 37% blocked at issue and 15% in vector ALU instructions;
+// 1000^3 bf16 8% busy, 46% waiting. Bank conflicts take a fifth of the LDS pipe's
+// active cycles, which are 9% (5%) of the waves'.
 //
 // Block tile kBM x kBN, K step 64, 256 lanes = 4 waves. A step's operands are
-// loaded into registers one step ahead, rounded there (fp32), and written to
+// loaded into registers one or two steps ahead, rounded there (fp32), and written to
 // one of two LDS stages in the fragment order of the packed layouts: per 32 k,
 // 1 KiB per 16 rows (columns), the 16-byte chunk of 8 k of row r, chunk c at
-// 256 c + 16 (r % 16 ^ swizzle). So each MFMA operand is one linear,
-// conflict-free ds_read_b128. A lane loads 8 k of a row of A per chunk; of B
+// 256 c + 16 (r % 16 ^ swizzle). So each MFMA operand is one linear
+// ds_read_b128. A lane loads 8 k of a row of A per chunk; of B
 // it loads 8 k rows of kCV neighbouring columns and transposes them in
 // registers (the fp32 form by choosing which two floats each packed conversion
 // takes), where the form before this one wrote B to LDS two bytes at a time.
@@ -119,10 +125,10 @@ __device__ __forceinline__ u16x4 round4(f32x4 v) {
 // is loaded element by element with zeros past K, as is everything when
 // n < kCV. Vector loads need element alignment only.
 //
-// On an MI355X, graph-timed, against the 128x128 kernel this one replaced:
-// 2048^3 fp32 operands as bf16 283.5 -> 42.7 us, 4096^3 1087 -> 242, 1000^3
-// (4 splits allowed) 45.2 -> 15.3; bf16 operands 1000^3 26.5 -> 12.0,
-// 3000x3001x1023 351 -> 58, 16x4096x4096 29.0 -> 11.2.
+// On an MI355X, one launch after another on one set of operands, against the
+// 128x128 kernel this one replaced: fp32 operands as bf16 2048^3 282 -> 39.0 us,
+// 4096^3 971 -> 224, 1000^3 (4 splits allowed) 43.7 -> 14.8; bf16 operands 1000^3
+// (likewise) 24.9 -> 9.8, 3000x3001x1023 346 -> 51.1, 16x4096x4096 27.7 -> 10.2.
 // kWM x kWN waves of a group tile the block's C tile; kG groups take every
 // kG-th K step each and are added at the end; kAhead: steps loaded ahead (in
 // registers); kBlocks: blocks per CU the register budget is cut for; kAcc: 1,
@@ -617,9 +623,10 @@ struct StagedPlan {
 // 128x128 tiles where they give at least four in five CUs one (the line of
 // split_k_splits, past which it asks for no ranges: a caller's own count runs
 // as given), else 64x64, or 32x64 for at most 32 rows; those in K ranges only
-// where they leave half the CUs idle (graph-timed on an MI355X, bf16 operands: 512x1024x2048, 128 tiles of
-// 64x64, 14.9 us in 2 ranges with their sum against 22.1 unsplit; 1000^3, 256
-// tiles, 12.5 us unsplit, where the 128x128 kernel in 4 ranges took 26.5).
+// where they leave half the CUs idle (on an MI355X, bf16 operands: 512x1024x2048,
+// 128 tiles of 64x64, 12.7 us in 2 ranges with their sum against 15.5 unsplit;
+// 1000^3, 256 tiles, 9.8 us unsplit, where the 128x128 kernel in 4 ranges took
+// 24.9).
 StagedPlan staged_plan(int m, int n, int k, int splits) {
     const long long cus = std::max(device_cus(), 1);
     const auto tiles = [&](int bm, int bn) {
@@ -658,14 +665,14 @@ int launch16(const void* a, const void* b, float* c, int m, int n, int k, hipStr
     };
     // The form of a tile, by operand type (us on an MI355X, K = 2048 or 2040).
     // 128x128: with at most one per CU two steps are loaded ahead (2048^2 fp32
-    // 42.7 against 48.5 with one; bf16 34.7 against 36.8), with more than one a
+    // 39.0 against 45.4 with one; bf16 30.5 against 32.9), with more than one a
     // second block per CU does better than the deeper prefetch (3072^2 fp32
-    // 100.4 against 114.3; bf16 80.8 against 85.6). Eight waves where the
-    // registers allow (bf16: 2048^2 34.7 against 44.3 with four; fp32 4096^2
-    // 141.8 on four waves against 154.9).
+    // 89.3 against 101.3; bf16 73 against 82.4). Eight waves where the
+    // registers allow (bf16: 2048^2 30.5 against 39.2 with four; fp32 4096^2
+    // 114.4 on four waves against 150).
     // 64x64, where the caller's split count leaves the order of adds open: two
     // groups of waves, each taking every other K step, where there is one tile
-    // per CU at most (bf16 1024^2 14.6 against 18.0; fp32 operands 768x768x4096
+    // per CU at most (bf16 1024^2 12.2 against 15.3; fp32 operands 768x768x4096
     // 35.1 against 39.6, 704x768x1024 12.1 against 12.7). The groups also keep
     // the error of the ranges asked for, up to seven where one range runs
     // (fp32 operands, 2-norm, 768x768x4096: 1.37e-7 in 7 ranges, 1.73e-7 with
