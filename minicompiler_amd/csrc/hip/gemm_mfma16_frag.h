@@ -189,11 +189,16 @@ __device__ __forceinline__ void mc_gemm16_frag(const unsigned short* __restrict_
 #pragma unroll
         for (int w = 1; w < kW; ++w) sum += red[w][t >> 6][t & 63];
         const int row = row_of(t), col = col_of(t);
-        if (row < m) {
+        if (row < m && col < n) {
             const unsigned at = static_cast<unsigned>(row) * static_cast<unsigned>(n) + static_cast<unsigned>(col);
+            if (n % 4 == 0 || col + 4 <= n) {  // a condition per chunk, as in fast_store
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (col + e < n) sum[e] = epilogue(sum[e], at + e);
+                for (int e = 0; e < 4; ++e) sum[e] = epilogue(sum[e], at + e);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 3; ++e)
+                    if (col + e < n) sum[e] = epilogue(sum[e], at + e);
+            }
         }
         sums[i] = sum;
     }

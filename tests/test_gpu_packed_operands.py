@@ -128,3 +128,23 @@ def test_graphs_on_ragged_sizes_fuse_and_match_float64(device, mc, oracle, kerne
         assert len(c.launch_nodes) == (1 if epilogue else 2)
         out = run_into_prefilled(mc, c, [x])[0].astype(np.float64)
         assert np.all(np.abs(out - want) <= bound), f"epilogue {epilogue}"
+
+
+# A residual read element by element at the matrix edge, its last element at the end of its buffer: N of each remainder
+# by 4, on 256x256, two-sum and small tiles; and B fed per run (whole chunks at every edge).
+@pytest.mark.parametrize("m,k,n,fed", [(1100, 70, 4000, False), (1031, 65, 4001, False), (2305, 40, 1794, False),
+                                       (1792, 130, 1791, False), (33, 64, 71, False), (300, 96, 130, False),
+                                       (300, 64, 264, True), (65, 128, 1000, True)])
+def test_fused_groups_at_the_edges(device, mc, oracle, m, k, n, fed):
+    text = (f"input x : f32[{m}, {k}]\ninput r : f32[{m}, {n}]\n"
+            + (f"input w : f32[{k}, {n}]\n" if fed else f"const w : f32[{k}, {n}] = uniform(seed=2, lo=-1, hi=1)\n")
+            + f"const b : f32[{n}] = uniform(seed=3, lo=-1, hi=1)\nh = matmul x, w\nhb = add h, b\ny = add hb, r\noutput y\n")
+    x, w, b = oracle.uniform(m * k, 1, -1.0, 1.0), oracle.uniform(k * n, 2, -1.0, 1.0), oracle.uniform(n, 3, -1.0, 1.0)
+    r = oracle.uniform(m * n, 4, -1.0, 1.0)
+    print(f"case fused edge {m}x{k}x{n} fed {fed}", flush=True)
+    exact, absdot = oracle.gemm_f64(oracle.round_bf16(x), oracle.round_bf16(w), m, k, n)
+    want = exact + np.tile(b.astype(np.float64), m) + r
+    c = mc.Compiled(text, options={"matmul": "tensor_core_bf16"})
+    assert len(c.launch_nodes) == 1
+    out = run_into_prefilled(mc, c, [x, r, w] if fed else [x, r])[0].astype(np.float64)
+    assert np.all(np.abs(out - want) <= gamma(k) * absdot + 4 * U32 * (np.abs(exact) + 2.0))
