@@ -809,11 +809,19 @@ ElementwiseKernel generate_column_kernel(const FusedProgram& program, const std:
 ElementwiseKernel generate_graph_kernel(const FusedProgram& program, const std::vector<Shape>& input_shapes,
                                         const Shape& out_shape, const CodegenOptions& options) {
     const std::size_t numel = num_elements(out_shape);
-    bool column = numel % 4 != 0;
+    bool column = numel % 4 != 0, odd_row = false;
     for (const Shape& s : input_shapes) {
-        const Access::Kind kind = classify_access(s, out_shape).kind;
-        column = column || kind == Access::Kind::Periodic || kind == Access::Kind::General;
+        const Access a = classify_access(s, out_shape);
+        column = column || a.kind == Access::Kind::Periodic || a.kind == Access::Kind::General;
+        odd_row = odd_row || (a.kind == Access::Kind::Periodic && a.period % 2 != 0);
     }
+    // Up to one vector for each lane of four waves on 256 CUs, a lane has one item
+    // and nothing to keep a row for; at an odd period the row's wrapped vector then
+    // costs more than the flat form's floats. A row, a value per row and a row
+    // again on an MI355X, flat / columns: [127, 129] 1.86 / 2.08 us, [128, 2047]
+    // 2.00 / 2.19, [2032, 129] 2.14 / 2.30; twice that count 3.40 / 2.62 at 129.
+    // One row alone is alike in both there, and so are rows of even period.
+    if (odd_row && options.items_per_lane == 0 && numel <= 262144) column = false;
     if (options.allow_vectorize && column && numel >= 1024) {
         return generate_column_kernel(program, input_shapes, out_shape, options);
     }

@@ -74,8 +74,8 @@ ElementwiseKernel generate_elementwise_kernel(const FusedProgram& program, const
 
 // The kernel a compiled graph runs for an elementwise node: the column form
 // (codegen.cpp, generate_column_kernel) for 1024 elements or more with a
-// broadcast input or a count that is not a multiple of 4, else
-// generate_elementwise_kernel's.
+// broadcast input or a count that is not a multiple of 4 (more than 262,144
+// with a row of odd period), else generate_elementwise_kernel's.
 ElementwiseKernel generate_graph_kernel(const FusedProgram& program, const std::vector<Shape>& input_shapes,
                                         const Shape& out_shape, const CodegenOptions& options = {});
 

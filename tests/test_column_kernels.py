@@ -107,3 +107,10 @@ def test_small_counts_scalars_and_whole_vectors_keep_the_flat_form(mc):
         assert ("vectors apart" in src) == column
         (flat,) = mc.Compiled(text, passes="none", backend="none", options={"vectorize": 0}).kernel_sources
         assert "vectors apart" not in flat
+
+
+def test_rows_of_odd_period_take_the_column_form_for_large_counts_only(mc):
+    for rows, cols, column in ((2032, 129, False), (2033, 129, True), (16, 250, True), (16, 129, False), (16384, 16, True)):
+        text = f"input x : f32[{rows}, {cols}]\ninput b : f32[{cols}]\ny = add x, b\noutput y\n"
+        (src,) = mc.Compiled(text, passes="none", backend="none").kernel_sources
+        assert ("vectors apart" in src) == column, (rows, cols)
