@@ -160,7 +160,9 @@ int mchip_f32_narrow_plan(int m, int n, int k, int max_splits, int cu_count, int
  * operands not 16-byte aligned (any float address). The ring's from K 64 and
  * N 4 on (MCHIP_RING_WIDE, MCHIP_RING_WIDE8 or MCHIP_RING_NONE; one block
  * per tile and split), the narrow body's as mchip_f32_narrow_plan decides
- * for N and K rounded up, from K 16 and N 4 on. Smaller ones stay on the
+ * for N and K rounded up (but 64x64 tiles in any number of ranges past K =
+ * 2048, or 32x64 tiles in their place where those fill the chip better), from
+ * K 16 and N 4 on. Smaller ones stay on the
  * two-stage body. They do not add splits in the launch. */
 int mchip_f32_ragged_ring_plan(int m, int n, int k, int depth, int cu_count, unsigned* grid, unsigned* block);
 int mchip_f32_ragged_narrow_plan(int m, int n, int k, int max_splits, int cu_count, int* shape, int* splits,

@@ -511,7 +511,28 @@ extern "C" int mchip_f32_ragged_narrow_plan(int m, int n, int k, int max_splits,
                                             int* k_split) {
     *shape = *splits = *k_split = 0;
     if (m < 1 || n < 4 || k < 16 || n > 0x7ffffff0 || k > 0x7ffffff0) return 0;
-    return mchip_f32_narrow_plan(m, (n + 3) / 4 * 4, (k + 15) / 16 * 16, max_splits, cu_count, 0, shape, splits, k_split);
+    if (!mchip_f32_narrow_plan(m, (n + 3) / 4 * 4, (k + 15) / 16 * 16, max_splits, cu_count, 0, shape, splits, k_split)) {
+        return 0;
+    }
+    if (*shape != MCHIP_NARROW_64X64) return 1;
+    // The exact plan's 64x64 tiles leave up to half of the CUs idle at some sizes,
+    // in its powers of two of ranges or in a second round nearly empty; the
+    // two-stage body in all the ranges asked for, which ran these sizes before,
+    // did not. So here: past K = 2048 as many ranges as fill the chip, or 32x64
+    // tiles unsplit where 64x64 ones would run unsplit on half of it; and 32x64
+    // tiles where 64x64 ones number up to 1.25 per CU. On an MI355X, the two-stage
+    // body / powers of two / so: 96x2192x8100 55.8 / 67.7 / 50.1 us (2 ranges
+    // become 3), 193x2240x4444 57.8 / 70.6 / 48.0 (140 tiles become 245 of 32x64),
+    // 618x1792x904 34.6 / 38.4 / 34.8 (280 become 560). Each of them adds sums.
+    const auto tiles = [&](int rows) { return static_cast<long long>((m + rows - 1) / rows) * ((n + 63) / 64); };
+    if (*splits == 1 && ((k > 2048 && tiles(32) <= cu_count) || (tiles(64) > cu_count && 4 * tiles(64) <= 5 * cu_count))) {
+        *shape = MCHIP_NARROW_32X64;
+    } else if (k > 2048) {
+        const long long s = std::max<long long>(1, std::min<long long>(max_splits, cu_count / tiles(64)));
+        *k_split = static_cast<int>((((k + s - 1) / s) + 15) / 16 * 16);
+        *splits = (k + *k_split - 1) / *k_split;
+    }
+    return 1;
 }
 
 extern "C" int mchip_narrow_rows(int shape) {

@@ -18,7 +18,9 @@ DOUBLE_BUFFERED = [(128, 129, 65), (129, 130, 95), (300, 131, 1023), (2100, 2049
                    (257, 4, 64), (130, 5, 70), (64, 300, 129)]
 SPLIT_K = [(1, 5, 17, 1), (16, 1001, 777, 6), (20, 70, 33, 1), (65, 513, 2049, 8), (33, 1030, 1000, 4),
            (1000, 1001, 1023, 4), (257, 515, 4097, 16), (512, 130, 130, 3), (200, 18, 1000, 15), (7, 6, 100, 4),
-           (1, 2048, 512, 8), (1, 516, 2048, 8), (17, 1000, 1023, 4), (128, 512, 144, 2), (31, 33, 129, 2)]
+           (1, 2048, 512, 8), (1, 516, 2048, 8), (17, 1000, 1023, 4), (128, 512, 144, 2), (31, 33, 129, 2),
+           # 64x64 tiles in three ranges, the last one short; 32x64 tiles in their place, K long and short
+           (96, 2192, 2084, 14), (128, 2181, 2051, 14), (200, 2181, 2050, 7), (618, 1797, 130, 3)]
 
 
 def check(mc, oracle, kernel, m, n, k, splits, offsets):
@@ -75,7 +77,8 @@ def test_infinities_and_nans_stay_in_their_row_and_column(device, mc, oracle, ke
 
 
 # A bias (periodic operand) and a residual (contiguous, its last element at the end of its buffer).
-@pytest.mark.parametrize("m,n,k", [(300, 131, 1023), (2100, 2050, 70), (20, 71, 500), (1, 1001, 1023), (129, 9, 66)])
+@pytest.mark.parametrize("m,n,k", [(300, 131, 1023), (2100, 2050, 70), (20, 71, 500), (1, 1001, 1023), (129, 9, 66),
+                                   (96, 2192, 2084)])
 @pytest.mark.parametrize("matmul", ["auto", "double_buffered", "split_k"])
 def test_fused_groups_at_the_matrix_edge(device, mc, oracle, m, n, k, matmul):
     print(f"case ragged fused {matmul} {m}x{n}x{k}", flush=True)

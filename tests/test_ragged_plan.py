@@ -46,3 +46,18 @@ def test_short_k_products_that_would_split_run_16x16_tiles(mc, m, n, k, splits, 
     f = mc.library().mchip_f32_narrow_plan
     out = [ctypes.c_int() for _ in range(3)]
     assert f(m, n, k, splits, 256, 0, *[ctypes.byref(x) for x in out]) and tuple(x.value for x in out) == want
+
+
+@pytest.mark.parametrize("m,n,k,splits,want", [
+    (96, 2192, 8100, 14, (4, 3, 2704)), (544, 464, 3896, 12, (4, 3, 1312)),   # 70 and 72 tiles: three ranges, not two
+    (96, 2192, 8100, 2, (4, 2, 4064)),                                        # no more than asked for
+    (193, 2240, 4444, 7, (0, 1, 4448)), (394, 1204, 3128, 6, (0, 1, 3136)),   # 140 and 133 tiles: 245 and 247 of 32x64
+    (333, 2112, 5516, 5, (4, 1, 5520)),                                       # 198 tiles: 363 of 32x64 are too many
+    (618, 1792, 904, 3, (0, 1, 912)),                                         # 280 tiles: 1.1 rounds
+    (1000, 1001, 1023, 4, (4, 1, 1024)), (2000, 1001, 1023, 2, (4, 1, 1024)),  # one and two whole rounds
+    (300, 424, 4968, 21, (0, 2, 2496)),                                       # 32x64 tiles to begin with
+])
+def test_ragged_64x64_tiles_fill_the_chip(mc, m, n, k, splits, want):
+    f = mc.library().mchip_f32_ragged_narrow_plan
+    out = [ctypes.c_int() for _ in range(3)]
+    assert f(m, n, k, splits, 256, *[ctypes.byref(x) for x in out]) and tuple(x.value for x in out) == want
