@@ -370,7 +370,8 @@ GemmEpilogueKernel generate_gemm_epilogue_kernel(const FusedProgram& program, st
         os << "\tmc_gemm_f32_mfma<true, " << (vectorized_operands ? "true" : "false") << ">(a, b, c, " << mnk
            << ", " << (constant ? std::to_string(fixed.k_split) : std::string("k_split")) << ", partial, epi);\n}\n\n";
     } else if (is_narrow_body(body)) {
-        os << "\tmc_gemm_f32_narrow<" << narrow_config(body) << ragged << ">(a, b, c, "
+        const bool sums = body == GemmBody::F32Narrow16x32 && fixed.ragged && fixed.k > kNarrowSumsK;
+        os << "\tmc_gemm_f32_narrow<" << (sums ? "McNarrow16x32Sums" : narrow_config(body)) << ragged << ">(a, b, c, "
            << mnk << ", " << split << ", partial, counters, epi);\n}\n\n";
     } else {
         const char* cfg = body == GemmBody::F32RingBig    ? "McRingBig"

@@ -106,6 +106,14 @@ using McNarrow16 = McNarrowCfg<1, 4, 4, 2, true>;
 using McNarrow32 = McNarrowCfg<2, 4, 4, 2, false>;
 using McNarrow16x64 = McNarrowCfg<1, 4, 4, 2, false>;
 using McNarrow16x32 = McNarrowCfg<1, 2, 4, 2, false>;
+// The ragged form's 16x32 tiles past K = kNarrowSumsK: they take over from up to
+// 31 ranges of the two-stage body, whose sums are more than four accumulators
+// from about K = 1750 on (2-norm error in ranges / with four / with eight:
+// 231x262x1677 1.93e-7 / 1.91e-7 / 1.44e-7, 74x1193x1815 1.95e-7 / 2.00e-7 /
+// 1.49e-7, 444x156x2047 1.96e-7 / 2.11e-7 / 1.57e-7; 157x693x334 1.75e-7 /
+// 1.00e-7 / 0.88e-7). Eight cost 0.05 to 0.2 us of 3.3 to 5.9 up to K = 1000
+// and 0.03 to 0.2 of 7.3 to 13.2 past 1536 (0.2 to 0.4 under a fused epilogue).
+using McNarrow16x32Sums = McNarrowCfg<1, 2, 4, 2, false, 16, 8>;
 // 64x64 tiles: each operand byte a wave loads feeds 64 MFMAs per 16 k
 // where 32x64 tiles feed 32 per 6 loads (1024^3 as 256 unsplit tiles). One
 // block per CU: its 96 KiB reduction array leaves no room for a second.
@@ -223,11 +231,9 @@ __device__ __forceinline__ void mc_gemm_f32_narrow(const float* __restrict__ a, 
     // many partial sums the rounding error is no larger. Relative error in
     // the 2-norm and time on an MI355X, the two-stage body / one accumulator
     // / these: 449x1263x1472 2.9e-7 39.1 us / 3.5e-7 29.0 us / 2.5e-7 30.6 us,
-    // 64x2032x1327 1.9e-7 19.0 us / 3.3e-7 8.7 us / 1.7e-7 8.7 us. 16x32 tiles
-    // take over from the most ranges and keep eight (256x261x2047, 22 ranges
-    // before: 1.97e-7, 2.11e-7 with four, 1.57e-7 with eight).
-    constexpr int kAcc =
-        Cfg::kAcc > 1 || !kRagged ? Cfg::kAcc : kRG * kVec <= 2 ? 8 : kRG * kVec <= 8 ? 4 : 2;
+    // 64x2032x1327 1.9e-7 19.0 us / 3.3e-7 8.7 us / 1.7e-7 8.7 us. (16x32 tiles
+    // with long K: McNarrow16x32Sums.)
+    constexpr int kAcc = Cfg::kAcc > 1 || !kRagged ? Cfg::kAcc : kRG * kVec <= 8 ? 4 : 2;
     mc_nw_f32x4 part_acc[kAcc][kRG][kVec] = {};
     // Loads of `units` groups from group g into x, then (after a scheduling
     // barrier: left to itself the scheduler interleaves each load with the

@@ -136,6 +136,7 @@ enum {
     MCHIP_NARROW_64X64 = 4,         /* 64x64 tiles */
     MCHIP_NARROW_16X16 = 5,         /* 16x16 tiles, 8 waves, unsplit */
 };
+enum { kNarrowSumsK = 1536 }; /* ragged 16x32 tiles keep more sums past this K (McNarrow16x32Sums) */
 int mchip_narrow_rows(int shape);
 int mchip_narrow_cols(int shape);
 

@@ -244,16 +244,21 @@ int device_cu_count() {
     return cus;
 }
 
+template <class Cfg, bool kRagged>
+void narrow_form(const float* a, const float* b, float* c, int m, int n, int k, hipStream_t s, int k_split, int depth,
+                 float* part, unsigned* counters) {
+    const dim3 grid(((n + Cfg::kCols - 1) / Cfg::kCols) * depth * ((m + Cfg::kRows - 1) / Cfg::kRows));
+    hipLaunchKernelGGL((matmul_narrow_f32<Cfg, kRagged>), grid, dim3(Cfg::kThreads), 0, s, a, b, c, m, n, k, k_split,
+                       depth, part, counters);
+}
+
 template <class Cfg>
 void narrow_kernel(const float* a, const float* b, float* c, int m, int n, int k, hipStream_t s, int k_split,
                    int depth, float* part, unsigned* counters, bool ragged) {
-    const dim3 grid(((n + Cfg::kCols - 1) / Cfg::kCols) * depth * ((m + Cfg::kRows - 1) / Cfg::kRows));
     if (ragged) {
-        hipLaunchKernelGGL((matmul_narrow_f32<Cfg, true>), grid, dim3(Cfg::kThreads), 0, s, a, b, c, m, n, k, k_split,
-                           depth, part, counters);
+        narrow_form<Cfg, true>(a, b, c, m, n, k, s, k_split, depth, part, counters);
     } else {
-        hipLaunchKernelGGL((matmul_narrow_f32<Cfg, false>), grid, dim3(Cfg::kThreads), 0, s, a, b, c, m, n, k, k_split,
-                           depth, part, counters);
+        narrow_form<Cfg, false>(a, b, c, m, n, k, s, k_split, depth, part, counters);
     }
 }
 
@@ -274,7 +279,13 @@ int launch_narrow(const float* a, const float* b, float* c, int m, int n, int k,
             narrow_kernel<McNarrow16>(a, b, c, m, n, k, s, k_split, depth, part, ctr, ragged);
             break;
         case MCHIP_NARROW_16X64: narrow_kernel<McNarrow16x64>(a, b, c, m, n, k, s, k_split, depth, part, ctr, ragged); break;
-        case MCHIP_NARROW_16X32: narrow_kernel<McNarrow16x32>(a, b, c, m, n, k, s, k_split, depth, part, ctr, ragged); break;
+        case MCHIP_NARROW_16X32:
+            if (ragged && k > kNarrowSumsK) {
+                narrow_form<McNarrow16x32Sums, true>(a, b, c, m, n, k, s, k_split, depth, part, ctr);
+            } else {
+                narrow_kernel<McNarrow16x32>(a, b, c, m, n, k, s, k_split, depth, part, ctr, ragged);
+            }
+            break;
         case MCHIP_NARROW_64X64: narrow_kernel<McNarrow64>(a, b, c, m, n, k, s, k_split, depth, part, ctr, ragged); break;
         case MCHIP_NARROW_16X16: narrow_kernel<McNarrow16x16>(a, b, c, m, n, k, s, k_split, depth, part, ctr, ragged); break;
         default: return hipErrorInvalidValue;

@@ -146,6 +146,7 @@ int main(int, char** argv) {
         narrow_sizes<McNarrow32>("32x64");
         narrow_sizes<McNarrow16x64>("16x64");
         narrow_sizes<McNarrow16x32>("16x32");
+        narrow_sizes<McNarrow16x32Sums>("16x32 with more sums");
         narrow_sizes<McNarrow64>("64x64");
         narrow_sizes<McNarrow16x16>("16x16");
     } else {

@@ -112,7 +112,8 @@ def test_graphs_past_the_small_tiles_have_the_bits_of_the_operators_two_ranges(d
 
 
 # FP32, N or K off the exact forms' steps, on the narrow tiles of each width that run one range where many are asked for.
-@pytest.mark.parametrize("m,n,k", [(256, 261, 2047), (250, 300, 1700), (512, 261, 2047), (1000, 1001, 1023), (64, 2032, 1327)])
+@pytest.mark.parametrize("m,n,k", [(256, 261, 2047), (250, 300, 1700), (231, 261, 1537), (231, 262, 1535),
+                                   (512, 261, 2047), (1000, 1001, 1023), (64, 2032, 1327)])
 def test_ragged_fp32_products_keep_the_error_of_the_ranges_they_were_asked_for(device, mc, oracle, m, n, k):
     a = oracle.uniform(m * k, 7, -1.0, 1.0).reshape(m, k)
     b = oracle.uniform(k * n, 8, -1.0, 1.0).reshape(k, n)

@@ -20,7 +20,9 @@ SPLIT_K = [(1, 5, 17, 1), (16, 1001, 777, 6), (20, 70, 33, 1), (65, 513, 2049, 8
            (1000, 1001, 1023, 4), (257, 515, 4097, 16), (512, 130, 130, 3), (200, 18, 1000, 15), (7, 6, 100, 4),
            (1, 2048, 512, 8), (1, 516, 2048, 8), (17, 1000, 1023, 4), (128, 512, 144, 2), (31, 33, 129, 2),
            # 64x64 tiles in three ranges, the last one short; 32x64 tiles in their place, K long and short
-           (96, 2192, 2084, 14), (128, 2181, 2051, 14), (200, 2181, 2050, 7), (618, 1797, 130, 3)]
+           (96, 2192, 2084, 14), (128, 2181, 2051, 14), (200, 2181, 2050, 7), (618, 1797, 130, 3),
+           # 16x32 tiles with four accumulators and, past K = 1536, with eight
+           (231, 261, 1536, 10), (231, 261, 1537, 10), (157, 693, 334, 5)]
 
 
 def check(mc, oracle, kernel, m, n, k, splits, offsets):
