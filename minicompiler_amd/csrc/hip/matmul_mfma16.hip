@@ -328,7 +328,9 @@ __global__ void __launch_bounds__(Cfg::kThreads, Cfg::kBlocks) matmul_mfma16_sta
     // condition, the compiler's wait for one set would wait for the sets
     // loaded after it too. What is left is at most one more step per group,
     // whole, partial or empty (zeros), loaded ahead as well where there are
-    // registers for it; with n < kCV every step is of that kind.
+    // registers for it; with n < kCV every step is of that kind. An empty one
+    // loads nothing (from fp32 768x768x320, one group's third step empty, 9.0 us
+    // with clamped loads, 7.6 without).
     constexpr int kAhead = Cfg::kAhead, kG = Cfg::kG;
     const int tiles = ke > kb ? (ke - kb + kBK - 1) / kBK : 0;
     const int full = whole_cols ? (ke - kb) / kBK : 0;
@@ -339,8 +341,10 @@ __global__ void __launch_bounds__(Cfg::kThreads, Cfg::kBlocks) matmul_mfma16_sta
     auto load_rest = [&](Regs& r, int i) {
         if (i * kG + grp < full) {
             load_whole(r, k_of(i));
-        } else {
+        } else if (kG == 1 || i * kG + grp < tiles) {
             load_part(r, k_of(i));
+        } else {
+            r = Regs{};
         }
     };
     Regs rest;
@@ -672,15 +676,20 @@ int launch16(const void* a, const void* b, float* c, int m, int n, int k, hipStr
     // 114.4 on four waves against 150).
     // 64x64, where the caller's split count leaves the order of adds open: two
     // groups of waves, each taking every other K step, where there is one tile
-    // per CU at most (bf16 1024^2 12.2 against 15.3; fp32 operands 768x768x4096
-    // 35.1 against 39.6, 704x768x1024 12.1 against 12.7). The groups also keep
-    // the error of the ranges asked for, up to seven where one range runs
-    // (fp32 operands, 2-norm, 768x768x4096: 1.37e-7 in 7 ranges, 1.73e-7 with
-    // one group of four accumulators, 1.21e-7 with two). fp32 operands in more
-    // than three ranges keep one group: four accumulators per range are enough
-    // sums, and a range has too few steps for two (256x256x2048 in 16 ranges
-    // 9.5 against 9.9).
+    // per CU at most (bf16 1024^2 12.2 against 15.3). fp32 operands are bound by
+    // the loads themselves and run one group, but where its four accumulators per
+    // range are fewer sums than the ranges asked for, and the ranges long enough
+    // for the error to show it. 2-norm error with one group and with two, of that
+    // in the ranges asked for, and us:
+    //   1 range, 768x768: bf16 K = 4096 1.26 and 0.89, 39.5 and 35.2; K = 576 0.99
+    //     and 0.89, 8.5 and 9.3; fp16 K = 448 1.06 and 0.94, 7.4 and 8.0;
+    //   2 ranges, 256x1400: bf16 K = 4095 1.06 and 0.82, 30.5 and 29.4; fp16 K =
+    //     2048 1.03 and 0.82, 15.8 and 15.3; K = 1536 0.96 with one;
+    //   3 ranges, 128x2176: fp16 K = 6144 1.00 and 0.78, 24.6 and 23.5; K = 4032
+    //     0.96 with one; bf16 K = 2048 0.88 and 0.79, 13.0 and 13.4.
     const long long cus = std::max(device_cus(), 1);
+    const int enough = p.depth == 1 ? (kBf16 ? 576 : 256) : p.depth == 2 ? 768 : 1344;
+    const bool more_sums = p.depth <= 3 && splits > 4 * p.depth && p.k_split > enough;
     if (p.bm == 128) {
         if constexpr (kF32In) {
             if (p.tiles <= cus) {
@@ -698,7 +707,7 @@ int launch16(const void* a, const void* b, float* c, int m, int n, int k, hipStr
     } else if (p.bm == 64) {
         if (splits <= 1) {
             run(Staged<64, 64, 2, 2, 1, 2, 2>{});
-        } else if (p.tiles > cus || (kF32In && p.depth > 3)) {
+        } else if (p.tiles > cus || (kF32In && !more_sums)) {
             run(Staged<64, 64, 2, 2, 1, 2, 2, 4>{});
         } else {
             run(Staged<64, 64, 2, 2, 2, 2, 1, 4>{});

@@ -41,10 +41,13 @@ def rounded(oracle, kernel, x):
     return rnd(x.reshape(-1)).reshape(x.shape).astype(np.float64)
 
 
-# 36 to 51 tiles of 128x128 (5 to 7 ranges asked for, none run), 13 to 25 (10 to 19 asked for, 2 to 4 run), few rows.
+# 36 to 51 tiles of 128x128 (5 to 7 ranges asked for, none run), 13 to 25 (10 to 19 asked for, 2 to 4 run), few rows;
+# last, both sides of the lengths from which fp32 operands run two groups of waves, in one, two and three ranges.
 @pytest.mark.parametrize("kernel", ["tensor_core_bf16", "tensor_core_f16"])
 @pytest.mark.parametrize("m,n,k", [(704, 768, 2048), (640, 832, 4096), (1024, 768, 4095), (640, 640, 4096),
-                                   (1664, 128, 4096), (32, 2048, 4096)])
+                                   (1664, 128, 4096), (32, 2048, 4096),
+                                   (96, 5440, 320), (768, 768, 448), (96, 5440, 576), (96, 5440, 577),
+                                   (256, 1400, 1536), (256, 1400, 1537), (128, 2176, 4032), (128, 2176, 4033)])
 def test_the_operator_keeps_the_error_of_the_ranges_it_was_asked_for(device, mc, oracle, kernel, m, n, k):
     a = oracle.uniform(m * k, 7, -1.0, 1.0).reshape(m, k)
     b = oracle.uniform(k * n, 8, -1.0, 1.0).reshape(k, n)
