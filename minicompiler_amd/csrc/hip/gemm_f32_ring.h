@@ -16,7 +16,7 @@
 // Requirements (checked by the host): K (and the split size) a multiple of
 // 32, N a multiple of 4, A, B, C and the partials 16-byte aligned, every
 // split non-empty; counters (when given): one zeroed unsigned per tile.
-// Rows past M read the last row and columns past N the tile's first chunk, so
+// Rows past M read the last row and columns past N the tile's last chunk, so
 // every load is in bounds; what they bring only reaches C elements that are
 // not stored.
 //
@@ -623,8 +623,8 @@ __device__ __forceinline__ void mc_gemm_f32_ring(const float* __restrict__ a, co
     // logical chunk that ^ 8 (k row / 16 % 2).
     constexpr int kLanesPerBRow = Cfg::kBRow / 16;
     // Offsets are from the unit's origin. Rows past M read row M - 1, columns past
-    // N the tile's first chunk: both at or past the origin, also where N is no
-    // multiple of 4 and a last tile has fewer than 4 columns.
+    // N the last 4, or the tile's first where N is no multiple of 4 and the last
+    // tile has fewer: all at or past the origin.
     auto fetch_of = [&](const McRingUnit& u) {
         McRingFetch<Cfg> f;
         f.a_rsrc = mc_ring_rsrc(a + static_cast<long long>(u.row0) * k + u.kb);
@@ -641,7 +641,7 @@ __device__ __forceinline__ void mc_gemm_f32_ring(const float* __restrict__ a, co
             const int kk = (Cfg::kFB * wave + i) * (1024 / Cfg::kBRow) + lane / kLanesPerBRow;
             const int g = (lane % kLanesPerBRow) ^ (8 * ((kk >> 4) & 1));
             int col = u.col0 + 4 * g;
-            if (col >= n) col = u.col0;
+            if (col >= n) col = n - 4 > u.col0 ? n - 4 : u.col0;
             f.b_off[i] = 4 * (kk * n + col - u.col0);
         }
         f.b_step = 4 * Cfg::kBK * n;

@@ -118,7 +118,7 @@ static void ring(const char* name, int m, int n, int k, int k_split) {
 template <class Cfg>
 static void narrow_sizes(const char* name) {
     constexpr int R = Cfg::kRows, C = Cfg::kCols;
-    for (int n : {C + 1, C + 2, C + 3, 2 * C - 1, C, C + 4})
+    for (int n : {C + 1, C + 2, C + 3, 2 * C - 1, C, C + 4, 4, 6})
         for (int k : {16, 17, 31, 33, 100}) narrow<Cfg, true>(name, Cfg::kStreamB ? R : R + 1, n, k, 16 * up(k, 16));
     narrow<Cfg, true>(name, R, C + 1, 200, 64);
     narrow<Cfg, true>(name, 1, C + 1, 129, 64);
