@@ -111,8 +111,9 @@ using McNarrow16x32 = McNarrowCfg<1, 2, 4, 2, false>;
 // from about K = 1750 on (2-norm error in ranges / with four / with eight:
 // 231x262x1677 1.93e-7 / 1.91e-7 / 1.44e-7, 74x1193x1815 1.95e-7 / 2.00e-7 /
 // 1.49e-7, 444x156x2047 1.96e-7 / 2.11e-7 / 1.57e-7; 157x693x334 1.75e-7 /
-// 1.00e-7 / 0.88e-7). Eight cost 0.05 to 0.2 us of 3.3 to 5.9 up to K = 1000
-// and 0.03 to 0.2 of 7.3 to 13.2 past 1536 (0.2 to 0.4 under a fused epilogue).
+// 1.00e-7 / 0.88e-7). Eight cost 0.02 to 0.2 us of 3.3 to 5.9 up to K = 1000
+// (0.2 to 0.4 under a fused epilogue) and 0.04 to 0.2 of 7.3 to 13.2 past 1536
+// (0.03 to 0.3).
 using McNarrow16x32Sums = McNarrowCfg<1, 2, 4, 2, false, 16, 8>;
 // 64x64 tiles: each operand byte a wave loads feeds 64 MFMAs per 16 k
 // where 32x64 tiles feed 32 per 6 loads (1024^3 as 256 unsplit tiles). One
